@@ -139,6 +139,7 @@ struct lsf_engine {
   lsf::StepArgs* dev_args = nullptr;  // library scratch: [0] E kernel, [1] H kernel arguments
   const lsf::StepArgs* args_override = nullptr;  // during lsf_step_noalloc: the arguments staged in `scratch`
   lsf::StepArgs host_args[2];          // lsf_step_noalloc: host source of the staged arguments (outlives the copy)
+  int flat[2] = {0, 0};                // planes per tile of the flat E [0] and H [1] kernels; 0: the row kernels
   int nb[2] = {0, 0}, nbp[2] = {0, 0};  // tiles of the E [0] and H [1] launches (and padded to a multiple of 8)
   bool dirty = true;                   // dev_args out of date
   bool launched = false;               // kernels may be reading dev_args
@@ -173,8 +174,29 @@ Tiling own_tiling(const lsf_engine* e) { return Tiling{e->ry, e->waves, e->xw, e
 // arrays); the single-pass kernel rounds 1 up to 2
 int pole_regs(const lsf_engine* e) { return e->n_ade > 0 ? e->max_poles : 0; }
 
+bool any_periodic(const lsf_engine* e) { return e->g.per[0] || e->g.per[1] || e->g.per[2]; }
+
+// Engines with a periodic axis take the flat kernels for the one-row, four-wavefront tile shapes (what the drivers
+// and the default pick), except for the E update of D-form nodes.
+bool flat_kernel(const lsf_engine* e, int field, const Tiling& t) {
+  return any_periodic(e) && !e->adjoint && t.ry == 1 && t.waves == lsf::FLAT_WAVES && (field == 1 || pole_regs(e) == 0);
+}
+
+int flat_lpr(const lsf_engine* e) { return (e->g.n[0] + lsf::FLAT_CELLS - 1) / lsf::FLAT_CELLS; }
+
+// Planes per tile of a flat launch over these engines: 4 once that still leaves 16 wavefronts per SIMD (a plane
+// carried in registers saves two of ten loads), else 1. Measured at 1 / 2 / 4 planes: one 76 x 61 x 256 complex cell
+// FIXME us per step, 12 cells of 50-98 x 50-98 x 256 FIXME us.
+int flat_planes(const lsf_engine* const* mem, int n) {
+  long long waves = 0;
+  for (int q = 0; q < n; ++q)
+    waves += ((long long)flat_lpr(mem[q]) * mem[q]->g.n[1] + 63) / 64 * mem[q]->g.n[2];
+  return waves >= 4 * 16384 ? 4 : 1;
+}
+
 // Kernel arguments of engine e for field 0 (E kernel) or 1 (H kernel) under tiling t.
-StepArgs make_args(const lsf_engine* e, int field, const Tiling& t) {
+// flat: planes per tile of the flat kernels, 0 for the row kernels.
+StepArgs make_args(const lsf_engine* e, int field, const Tiling& t, int flat) {
   StepArgs a{};
   a.g = e->g;
   a.E = e->E;
@@ -202,14 +224,17 @@ StepArgs make_args(const lsf_engine* e, int field, const Tiling& t) {
   // the E kernel with pole state marches twice the z chunk (320^3, 10 % 3-pole nodes: E kernel 451 us at 8 planes
   // per tile, 442 us at 16; H kernel 269 us at 8, 276 us at 16)
   a.zc = field == 0 && !e->adjoint && pole_regs(e) > 0 ? 2 * t.zc : t.zc;
+  if (flat) {
+    a.zc = flat;
+    a.lpr = flat_lpr(e);
+    a.tiles_x = (int)(((long long)a.lpr * e->g.n[1] + 64 * t.waves - 1) / (64 * t.waves));
+    a.tiles_y = 1;
+  }
   const int tiles_z = (e->g.n[2] + a.zc - 1) / a.zc;
   a.nb = a.tiles_x * a.tiles_y * tiles_z;
   a.nbp = (a.nb + 7) / 8 * 8;
   return a;
 }
-
-bool any_periodic(const lsf_engine* e) { return e->g.per[0] || e->g.per[1] || e->g.per[2]; }
-
 
 void set_parity(lsf_engine* e, int p) {
   e->parity = p;
@@ -358,7 +383,8 @@ int sync_args(lsf_engine* e) {
   else if (e->launched) rc = hip_check(hipDeviceSynchronize(), "synchronize before an argument update");
   if (rc) return rc;
   const Tiling t = own_tiling(e);
-  const StepArgs h[2] = {make_args(e, 0, t), make_args(e, 1, t)};
+  for (int f = 0; f < 2; ++f) e->flat[f] = flat_kernel(e, f, t) ? flat_planes(&e, 1) : 0;
+  const StepArgs h[2] = {make_args(e, 0, t, e->flat[0]), make_args(e, 1, t, e->flat[1])};
   rc = hip_check(hipMemcpy(e->dev_args, h, sizeof h, hipMemcpyHostToDevice), "kernel argument upload");
   if (rc) return rc;
   for (int f = 0; f < 2; ++f) {
@@ -406,6 +432,7 @@ lsf::KLaunch own_launch(lsf_engine* e, int field) {
   L.per = any_periodic(e) ? 1 : 0;
   L.mat = e->mid ? 1 : 0;
   L.np = pole_regs(e);
+  L.flat = e->flat[field] > 0;
   return L;
 }
 
@@ -1246,8 +1273,10 @@ int lsf_step_noalloc(lsf_engine* e, int n, void* stream) {
   if (int rc = scratch_address(&p)) return rc;
   hipStream_t s = (hipStream_t)stream;
   const Tiling t = own_tiling(e);
-  e->host_args[0] = make_args(e, 0, t);
-  e->host_args[1] = make_args(e, 1, t);
+  for (int f = 0; f < 2; ++f) {
+    e->flat[f] = flat_kernel(e, f, t) ? flat_planes(&e, 1) : 0;
+    e->host_args[f] = make_args(e, f, t, e->flat[f]);
+  }
   for (int f = 0; f < 2; ++f) {
     e->nb[f] = e->host_args[f].nb;
     e->nbp[f] = e->host_args[f].nbp;
@@ -1536,8 +1565,9 @@ int build_groups(Level& L, const Tiling& t, int grid_blocks, std::vector<void*>&
       if (g.adj) tg.xw = 64;
       std::vector<StepArgs> args;
       std::vector<int> counts;
+      const int flat = flat_kernel(g.mem[0], field, tg) ? flat_planes(g.mem.data(), (int)g.mem.size()) : 0;
       for (lsf_engine* e : g.mem) {
-        args.push_back(make_args(e, field, tg));
+        args.push_back(make_args(e, field, tg, flat));
         counts.push_back(args.back().nb);
       }
       void* da = nullptr;
@@ -1554,6 +1584,7 @@ int build_groups(Level& L, const Tiling& t, int grid_blocks, std::vector<void*>&
       g.L.per = g.per;
       g.L.mat = g.mat;
       g.L.np = g.np;
+      g.L.flat = flat > 0;
     }
   }
   return LSF_OK;

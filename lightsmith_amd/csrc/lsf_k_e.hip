@@ -18,6 +18,8 @@ constexpr bool PER = LSF_E_PER != 0;
 
 template <int RY, int W, int XW, int NP>
 void go(const KLaunch& L, hipStream_t s) {
+  if constexpr (PER && NP == 0 && RY == 1 && W == FLAT_WAVES) return;  // the flat kernels' (lsf_flat.h)
+  else
   if (L.grid < L.sc.n_pad)
     hipLaunchKernelGGL((k_update_e<TE, LSF_E_MAT, RY, W, XW, PER, NP, true>), dim3(L.grid), dim3(64 * W), 0, s,
                        L.args, L.sc);

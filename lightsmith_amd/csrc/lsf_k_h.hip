@@ -16,6 +16,8 @@ using TH = std::conditional_t<LSF_H_CPLX != 0, c32, float>;
 
 template <int RY, int W, int XW, bool PER>
 void go(const KLaunch& L, hipStream_t s) {
+  if constexpr (PER && RY == 1 && W == FLAT_WAVES) return;  // the flat kernels' (lsf_flat.h)
+  else
   if (L.grid < L.sc.n_pad)
     hipLaunchKernelGGL((k_update_h<TH, RY, W, XW, PER, true>), dim3(L.grid), dim3(64 * W), 0, s, L.args, L.sc);
   else

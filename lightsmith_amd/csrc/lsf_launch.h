@@ -18,6 +18,7 @@ struct KLaunch {
   int per;               // some axis periodic
   int mat;               // E: 1 = packed material ids, 0 = dense coefficients
   int np;                // E: pole registers (0 or the engine's max_poles, 1 to 4)
+  int flat = 0;          // the flat kernels (lsf_flat.h) instead of the row kernels
 };
 
 // The tile shapes (rows per lane, wavefronts per block, x cells per row) with compiled kernels.
@@ -39,6 +40,12 @@ void launch_update_h_c(const KLaunch& L, hipStream_t s);
 LSF_E_LAUNCHERS(LSF_DECLARE_E)
 #undef LSF_DECLARE_E
 
+// the flat kernels of periodic engines without D-form nodes in the E update (lsf_flat.h): cells per lane and
+// wavefronts per block
+constexpr int FLAT_CELLS = 2, FLAT_WAVES = 4;
+void launch_flat_h(const KLaunch& L, hipStream_t s);
+void launch_flat_e(const KLaunch& L, hipStream_t s);
+
 // the single-pass step (real fields, no periodic axes, one row per wavefront, 64 x cells): lsf_k_fused.hip
 struct FusedArgs;
 // The tiles are split three ways by the CPML axes they touch (their halos included): none, x only, any other;
@@ -57,11 +64,13 @@ void launch_adjoint_h(const KLaunch& L, hipStream_t s);
 void launch_adjoint_e(const KLaunch& L, hipStream_t s);
 
 inline void launch_update_h(const KLaunch& L, hipStream_t s) {
+  if (L.flat) return launch_flat_h(L, s);
   if (L.cplx) launch_update_h_c(L, s);
   else launch_update_h_f(L, s);
 }
 
 inline void launch_update_e(const KLaunch& L, hipStream_t s) {
+  if (L.flat) return launch_flat_e(L, s);
 #define LSF_PICK_E(T, M, P) \
   if ((L.cplx != 0) == (#T[0] == 'c') && L.mat == M && (L.per != 0) == (P != 0)) return launch_update_e_##T##M##P(L, s);
   LSF_E_LAUNCHERS(LSF_PICK_E)

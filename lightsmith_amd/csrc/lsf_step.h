@@ -45,6 +45,7 @@ struct StepArgs {
   long long* counter;
   int tick;
   int tiles_x, tiles_y, zc, nb, nbp;
+  int lpr;               // lanes per x row of the flat kernels (tiles_x: their tiles per plane)
 };
 
 // The tiles of one launch: every member's tiles laid end to end.
@@ -704,8 +705,36 @@ __device__ __forceinline__ void e_tile(const StepArgs& a, int t, const float* ta
   }
 }
 
-// Each member's tile 0 advances its step counter: counter[1] = n, counter[0] = n + 1 (engine.py:678). The LDS
-// tables (indexed material, D-form media) are loaded again whenever the block moves to another member.
+// A member's tile 0 advances its step counter: counter[1] = n, counter[0] = n + 1 (engine.py:678).
+__device__ __forceinline__ void tick_counter(const StepArgs& a, int lt) {
+  if (a.tick && lt == 0 && threadIdx.x == 0) {
+    long long* cnt = (long long*)as_global(a.counter);
+    const long long n = cnt[0];
+    cnt[1] = n;
+    cnt[0] = n + 1;
+  }
+}
+
+// A member's LDS tables (indexed material, D-form media); `again`: the block held another member's before.
+template <int MAT, int WAVES, int NP>
+__device__ __forceinline__ void load_tables(const StepArgs& a, bool again, float* tab, float4* med_tab) {
+  if (again) __syncthreads();  // the previous member's readers are done
+  if (MAT == 1)
+    for (int q = threadIdx.x; q < 256; q += 64 * WAVES) tab[q] = ((const float*)as_global(a.mtab))[q];
+  if (NP > 0) {
+    const float* src = (const float*)as_global(a.media);
+    const int per = NP + 1, n = a.n_media_floats / a.media_stride;
+    for (int q = threadIdx.x; q < n * per; q += 64 * WAVES) {
+      const float* s = src + (q / per) * a.media_stride;
+      const int p = q % per - 1;
+      med_tab[q] = p < 0 ? make_float4(s[0], s[1], 0.f, 0.f)
+                         : make_float4(s[2 + 3 * p], s[3 + 3 * p], s[4 + 3 * p], 0.f);
+    }
+  }
+  __syncthreads();
+}
+
+// The LDS tables are loaded again whenever the block moves to another member.
 template <class T, int MAT, int RY, int WAVES, int XW, bool PER, int NP, bool LOOP>
 __global__ void __launch_bounds__(64 * WAVES) k_update_e(const StepArgs* __restrict__ args, Sched sc) {
   __shared__ float tab[MAT == 1 ? 256 : 1];
@@ -720,27 +749,9 @@ __global__ void __launch_bounds__(64 * WAVES) k_update_e(const StepArgs* __restr
     int m, lt;
     member_of(sc, t, m, lt);
     const StepArgs& a = args[m];
-    if (a.tick && lt == 0 && threadIdx.x == 0) {
-      long long* cnt = (long long*)as_global(a.counter);
-      const long long n = cnt[0];
-      cnt[1] = n;
-      cnt[0] = n + 1;
-    }
+    tick_counter(a, lt);
     if ((MAT == 1 || NP > 0) && m != cur) {
-      if (cur >= 0) __syncthreads();  // the previous member's readers are done
-      if (MAT == 1)
-        for (int q = threadIdx.x; q < 256; q += 64 * WAVES) tab[q] = ((const float*)as_global(a.mtab))[q];
-      if (NP > 0) {
-        const float* src = (const float*)as_global(a.media);
-        const int per = NP + 1, n = a.n_media_floats / a.media_stride;
-        for (int q = threadIdx.x; q < n * per; q += 64 * WAVES) {
-          const float* s = src + (q / per) * a.media_stride;
-          const int p = q % per - 1;
-          med_tab[q] = p < 0 ? make_float4(s[0], s[1], 0.f, 0.f)
-                             : make_float4(s[2 + 3 * p], s[3 + 3 * p], s[4 + 3 * p], 0.f);
-        }
-      }
-      __syncthreads();
+      load_tables<MAT, WAVES, NP>(a, cur >= 0, tab, med_tab);
       cur = m;
     }
     e_tile<T, MAT, RY, WAVES, XW, PER, NP>(a, lt, tab, med_tab);
