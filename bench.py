@@ -505,7 +505,7 @@ def main() -> int:
                     "frac": round(achieved / HBM_PEAK_GBS, 4),
                     "traffic": None if traffic is None else traffic.get("bytes_per_step"),
                     "traffic_source": traffic_src,
-                    "kernel": ("k_step_fused (one time step's bulk update in a single pass)" if h_ms == 0.0 else
+                    "kernel": ("k_pass (one time step's bulk update in a single pass)" if h_ms == 0.0 else
                                "k_update_h + k_update_e (one time step's bulk update)"),
                     "algorithmic_bytes_per_step": int(bytes_["total"]),
                     "kernel_us": {"h": round(h_ms * 1e3, 2), "e": round(e_ms * 1e3, 2)},

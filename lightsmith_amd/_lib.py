@@ -58,6 +58,8 @@ _SIGNATURES = {
     "lsf_add_tensor_group": [c_vp, c_i64, c_vp, c_vp, c_i64, c_vp, c_vp, c_vp, c_vp, c_int, c_int, c_vp, c_vp, c_vp,
                              c_vp, c_vp],
     "lsf_set_fused": [c_vp, c_vp, c_vp, ctypes.POINTER(c_vp)],
+    "lsf_set_pair": [c_vp, c_vp, c_vp, ctypes.POINTER(c_vp)],
+    "lsf_can_pair": [c_vp],
     "lsf_parity": [c_vp],
     "lsf_set_adjoint": [c_vp, c_int],
     "lsf_add_tape": [c_vp, c_i64, c_vp, c_vp, c_i64, c_vp],

@@ -13,8 +13,8 @@
 #include <vector>
 
 #include "lsf.h"
-#include "lsf_fused.h"
 #include "lsf_launch.h"
+#include "lsf_pass.h"
 #include "lsf_sparse.h"
 
 using lsf::c32;
@@ -145,19 +145,18 @@ struct lsf_engine {
   bool launched = false;               // kernels may be reading dev_args
   int held = 0;                        // batches holding this engine (its configuration is then frozen)
   int adjoint = 0;                     // steps the adjoint (transposed, time-reversed) update
-  // single-pass stepping: both field buffers and H-side psi sets, the parity of the current ones
+  // single-pass stepping (lsf_pass.h): both buffer sets; set 0 is current whenever the host has control
   void* Ebuf[2] = {nullptr, nullptr};
   void* Hbuf[2] = {nullptr, nullptr};
-  void* psiH[2][3][3] = {};            // [parity][axis][component]
-  int parity = 0;
-  bool fused_set = false;              // second buffers given (lsf_set_fused)
-  bool use_fused = false;              // the single-pass kernel steps this engine (decided at sync_args)
-  lsf::FusedArgs* dev_fused = nullptr; // library scratch: [parity]
-  int* dev_tiles = nullptr;            // single-pass tile lists by CPML class, back to back
-  int fused_count[3] = {0, 0, 0};
-  hipGraph_t graph2 = nullptr;         // the chunk graph starting at the other parity (odd strides)
-  hipGraphExec_t exec2 = nullptr;
-  int graph_parity = 0, graph_stride = 0;
+  void* psiH[2][3][3] = {};            // [set][axis][component]
+  bool pair_set = false;               // the second set is given (lsf_set_pair, lsf_set_fused)
+  bool asked_fused = false;            // by lsf_set_fused
+  bool passing = false;                // launching the operations that follow a pass
+  bool use_pass = false;               // pairs of steps run as single passes (decided at sync_args)
+  lsf::PassArgs* dev_pass = nullptr;   // library scratch: [set read]
+  lsf::DChunk* dform = nullptr;        // library scratch: D-form chunk table
+  int pass_nb = 0;                     // tiles of a pass
+  int pass_z[2] = {0, 0};              // planes [0], [1) in no z slab
 };
 
 namespace {
@@ -170,8 +169,7 @@ struct Tiling {
 
 Tiling own_tiling(const lsf_engine* e) { return Tiling{e->ry, e->waves, e->xw, e->zc}; }
 
-// pole registers of the E kernel instantiation for this engine: its max_poles (the slot stride of the pole
-// arrays); the single-pass kernel rounds 1 up to 2
+// pole registers of the kernel instantiation for this engine: its max_poles (the slot stride of the pole arrays)
 int pole_regs(const lsf_engine* e) { return e->n_ade > 0 ? e->max_poles : 0; }
 
 bool any_periodic(const lsf_engine* e) { return e->g.per[0] || e->g.per[1] || e->g.per[2]; }
@@ -186,7 +184,7 @@ int flat_lpr(const lsf_engine* e) { return (e->g.n[0] + lsf::FLAT_CELLS - 1) / l
 
 // Planes per tile of a flat launch over these engines: 4 once that still leaves 16 wavefronts per SIMD (a plane
 // carried in registers saves two of ten loads), else 1. Measured at 1 / 2 / 4 planes: one 76 x 61 x 256 complex cell
-// FIXME us per step, 12 cells of 50-98 x 50-98 x 256 FIXME us.
+// 55 / 67 / 75 us per step, 12 cells of 50-98 x 50-98 x 256 521 / 516 / 515 us.
 int flat_planes(const lsf_engine* const* mem, int n) {
   long long waves = 0;
   for (int q = 0; q < n; ++q)
@@ -236,137 +234,154 @@ StepArgs make_args(const lsf_engine* e, int field, const Tiling& t, int flat) {
   return a;
 }
 
-void set_parity(lsf_engine* e, int p) {
-  e->parity = p;
+// Make buffer set p the one that launches read (E, H and the H-side psi).
+void use_set(lsf_engine* e, int p) {
   e->E = e->Ebuf[p];
   e->H = e->Hbuf[p];
   for (int ax = 0; ax < 3; ++ax)
     for (int c = 0; c < 3; ++c) e->pml[1][ax].psi[c] = e->psiH[p][ax][c];
 }
 
+// Operations that need H of the step before E is updated. The design tape is not one: H^{n+1/2} is still there after
+// the pass.
 bool has_h_phase_ops(const lsf_engine* e) {
   for (const Op& o : e->ops)
-    if (o.phase <= LSF_PH_ADVANCE_H || o.phase == LSF_PH_BEFORE_H) return true;
+    if ((o.phase <= LSF_PH_ADVANCE_H || o.phase == LSF_PH_BEFORE_H) && o.kind != OP_TAPE) return true;
   return false;
 }
 
-// elements from the first to the second psi array of (field, axis) when they are contiguous, else -1
-long long psi_gap(const lsf_engine* e, int field, int ax, int parity_set) {
+// elements from the first to the second H-side psi array of an axis when they are contiguous, else -1
+long long psi_gap(const lsf_engine* e, int ax) {
   const int c1 = ax == 0 ? 1 : 0, c2 = ax == 2 ? 1 : 2;
-  void* const* ps = field == 0 ? e->pml[0][ax].psi : e->psiH[parity_set][ax];
-  const long long ns = e->pml[field][ax].ns;
-  long long size = ns;
+  void* const* ps = e->psiH[0][ax];
+  long long size = e->pml[1][ax].ns;
   for (int a = 0; a < 3; ++a)
     if (a != ax) size *= e->g.n[a];
   if (!ps[c1] || !ps[c2]) return -1;
   return ((const char*)ps[c2] - (const char*)ps[c1]) == size * (long long)sizeof(float) ? size : -1;
 }
 
-bool fused_eligible(const lsf_engine* e) {
-  if (!e->fused_set || e->cplx || any_periodic(e) || e->adjoint || e->ry != 1 || e->xw != 64 || has_h_phase_ops(e))
+// Whether the single pass can step an engine: real fields on cubic cells, no periodic axes, the boxes of a grid without
+// mirror planes, no work between the H and the E update, a one-row, four-wavefront tile shape (the default and what the
+// drivers choose; another shape asks for the row kernels) and components below 4 GB (32-bit offsets).
+bool pass_eligible(const lsf_engine* e) {
+  if (!e->pair_set || e->cplx || any_periodic(e) || e->adjoint || e->ry != 1 || e->waves != lsf::PASS_WAVES ||
+      has_h_phase_ops(e))
     return false;
-  // the kernel assumes the stepped boxes of a grid without periodic axes or mirror planes
-  for (int c = 0; c < 3; ++c)
+  for (int c = 0; c < 3; ++c) {
+    if (e->g.s[c] != 1.f) return false;
     for (int ax = 0; ax < 3; ++ax) {
       const int n = e->g.n[ax];
       if (e->g.rE[c][ax][0] != (ax == c ? 0 : 1) || e->g.rE[c][ax][1] != n - 1) return false;
       if (e->g.rH[c][ax][0] != 0 || e->g.rH[c][ax][1] != (ax == c ? n : n - 1)) return false;
     }
-  const long long lim = 1LL << 32;  // the kernel addresses fields and psi blocks with 32-bit byte offsets
-  if (3 * e->g.N * 4 >= lim) return false;
-  for (int f = 0; f < 2; ++f)
-    for (int ax = 0; ax < 3; ++ax)
-      if (e->pml[f][ax].prof)
-        for (int p = 0; p < (f == 1 ? 2 : 1); ++p) {
-          const long long gap = psi_gap(e, f, ax, p);
-          if (gap < 0 || 2 * gap * 4 >= lim) return false;
-        }
-  return true;
+  }
+  return e->g.N < (1ll << 30);
 }
 
-lsf::FusedArgs fused_args(const lsf_engine* e, int p) {
-  lsf::FusedArgs a{};
+// Whether it is also the faster step. The pass moves fewer bytes but over two sets of E, H and H-side psi, so it gains
+// while both sets stay in the 256 MB memory-side cache, loses where only one does, and gains again where neither does
+// and it has pole state or rows off the 64-byte lines (its wavefronts cross row ends, the row kernels' do not). Measured
+// on boxes with 8 CPML cells, us per step, two kernels -> pass: 128 x 110 x 100, 3 poles 43 -> 32; 131 x 117 x 150 56 ->
+// 40; 192 x 160 x 128, 1 pole 73 -> 70 (both sets 240 MB); 200 x 160 x 140 81 -> 90 (182 and 300 MB); 514 x 96 x 80 77 ->
+// 89 (178 and 282 MB); 239 x 201 x 181, 2 poles 223 -> 177; 255 x 257 x 250, none 334 -> 308; 256^3, none 310 -> 309, 2
+// poles 389 -> 357; 320^3, none 576 -> 597, 3 poles 691 -> 667.
+bool pass_pays(const lsf_engine* e) {
+  const long long N = e->g.N, cache = 256ll << 20;
+  long long psi[2] = {0, 0};
+  for (int f = 0; f < 2; ++f)
+    for (int ax = 0; ax < 3; ++ax)
+      if (e->pml[f][ax].prof) psi[f] += 8 * (N / e->g.n[ax]) * e->pml[f][ax].ns;
+  const long long one = (24 + (e->mid ? 4 : 12)) * N + psi[0] + psi[1] + 8 * e->n_ade * (long long)pole_regs(e);
+  const long long both = one + 24 * N + psi[1];
+  if (both <= cache) return true;
+  return one > cache && (pole_regs(e) > 0 || e->g.n[0] % 16 != 0);
+}
+
+// Planes per tile of a pass. A tile begins with H of the plane below it, so more planes save work, while fewer make
+// tiles whose cells the caches still hold for their neighbours, and D-form rounds hide more of the first. Measured, us per
+// step at 2 / 4 / 8 / 16 planes: no poles, 120 x 110 x 100 27 / 29 / 27 / 32, 200 x 160 x 140 85 / 90 / 93 / 106, 256^3
+// 312 / 309 / 330 / 348; 2 poles per D-form node, 240 x 200 x 180 189 / 175 / 183 / 204, 256^3 399 / 358 / 357 / 379; 1
+// pole, 400 x 300 x 260 664 / 578 / 558 / 592. Small grids take fewer, down to one, while the blocks number less than
+// four per compute unit (40 x 36 x 32, 3 poles: 13.2 at 1, 15.4 at 2, the step's dipole and sampling included).
+int pass_planes(const lsf_engine* e, int tiles_p) {
+  int z = pole_regs(e) == 0 ? 2 : e->g.N >= (12ll << 20) ? 8 : 4;
+  while (z > 1 && (long long)tiles_p * ((e->g.n[2] + z - 1) / z) < 1024) z /= 2;
+  return z;
+}
+
+lsf::PassArgs pass_args(const lsf_engine* e, int set) {
+  lsf::PassArgs a{};
   a.g = e->g;
-  a.E_in = (const float*)e->Ebuf[p];
-  a.H_in = (const float*)e->Hbuf[p];
-  a.E_out = (float*)e->Ebuf[p ^ 1];
-  a.H_out = (float*)e->Hbuf[p ^ 1];
+  a.E_in = (const float*)e->Ebuf[set];
+  a.H_in = (const float*)e->Hbuf[set];
+  a.E_out = (float*)e->Ebuf[set ^ 1];
+  a.H_out = (float*)e->Hbuf[set ^ 1];
   a.cbd = e->cbd;
   a.mid = e->mid;
   a.mtab = e->mtab;
   for (int ax = 0; ax < 3; ++ax) {
-    const int c1 = ax == 0 ? 1 : 0;
-    a.prof[0][ax] = e->pml[0][ax].prof;
-    a.prof[1][ax] = e->pml[1][ax].prof;
-    a.psiE[ax] = (float*)e->pml[0][ax].psi[c1];
-    a.psiHi[ax] = (const float*)e->psiH[p][ax][c1];
-    a.psiHo[ax] = (float*)e->psiH[p ^ 1][ax][c1];
     for (int f = 0; f < 2; ++f) {
-      a.psz[f][ax] = e->pml[f][ax].prof ? psi_gap(e, f, ax, 0) : 0;
-      for (int c = 0; c < 3; ++c) a.pso[f][ax][c] = c == ax ? 0u : (unsigned)(lsf::psi_slot(c, ax) * a.psz[f][ax] * 4);
+      a.prof[f][ax] = e->pml[f][ax].prof;
       a.ns[f][ax] = e->pml[f][ax].ns;
-      a.has_k[f][ax] = e->pml[f][ax].has_k;
+    }
+    for (int c = 0; c < 3; ++c) {
+      a.psiE[ax][c] = (float*)e->pml[0][ax].psi[c];
+      a.psiHi[ax][c] = (const float*)e->psiH[set][ax][c];
+      a.psiHo[ax][c] = (float*)e->psiH[set ^ 1][ax][c];
     }
   }
-  a.chunk_base = e->chunk_base;
+  a.zlo = e->pass_z[0];
+  a.zhi = e->pass_z[1];
+  a.dform = e->dform;
   a.P = e->P;
   a.nchunk = (e->g.n[0] + 31) / 32;
-  a.max_poles = e->max_poles;
   a.media_stride = 2 + 3 * e->max_poles;
   a.n_media_floats = e->n_ade > 0 ? e->n_media * (2 + 3 * e->max_poles) : 0;
   a.media = e->media;
   a.counter = e->counter;
   a.tick = e->tick;
-  a.tiles_x = (e->g.n[0] + 63) / 64;
-  a.tiles_y = (e->g.n[1] + e->waves - 1) / e->waves;  // one row per wavefront
-  a.zc = e->zc;
+  const long long cells = (long long)e->g.n[0] * e->g.n[1];
+  const int per_block = lsf::PASS_OWN * lsf::PASS_WAVES;
+  a.tiles_p = (int)((cells + per_block - 1) / per_block);
+  a.zc = pass_planes(e, a.tiles_p);
   return a;
 }
 
-// The single-pass tiles in three lists by the CPML axes they touch: a tile reads psi on the x span [x0 - 1, x0 + 64),
-// the rows [j0 - 1, j0 + waves) and the planes [z0 - 1, z1) (the halo cells it recomputes included). Lists: no
-// CPML, x CPML only, any other.
-int fused_tiles(lsf_engine* e, const lsf::FusedArgs& a) {
-  const int n[3] = {e->g.n[0], e->g.n[1], e->g.n[2]};
-  std::vector<char> slab[3];
-  for (int ax = 0; ax < 3; ++ax) {
-    slab[ax].assign(n[ax], 0);
-    for (int f = 0; f < 2; ++f) {
-      if (!e->pml[f][ax].prof) continue;
-      std::vector<float4> pr(n[ax]);
-      const int rc = hip_check(hipMemcpy(pr.data(), e->pml[f][ax].prof, n[ax] * sizeof(float4), hipMemcpyDeviceToHost),
-                               "CPML profile read");
-      if (rc) return rc;
-      for (int q = 0; q < n[ax]; ++q)
-        if ((int)pr[q].w >= 0) slab[ax][q] = 1;
-    }
+// Arguments of the single pass, and the D-form chunk table.
+int sync_pass(lsf_engine* e, const StepArgs& ea) {
+  int rc = LSF_OK;
+  if (pole_regs(e) > 0) {
+    const long long n = 3ll * ea.nchunk * e->g.n[1] * e->g.n[2];
+    if (!e->dform) rc = hip_check(hipMalloc(&e->dform, sizeof(lsf::DChunk) * n), "hipMalloc D-form chunk table");
+    if (!rc) rc = hip_check(hipDeviceSynchronize(), "synchronize before the D-form chunk table");
+    if (rc) return rc;
+    lsf::launch_dform_chunks(ea, e->dform, n, nullptr);
+    if ((rc = hip_check(hipStreamSynchronize(nullptr), "D-form chunk table"))) return rc;
   }
-  auto touches = [&](int ax, int lo, int hi) {  // any slab node in [lo, hi) (clamped to the grid)
-    for (int q = std::max(lo, 0); q < std::min(hi, n[ax]); ++q)
-      if (slab[ax][q]) return true;
-    return false;
-  };
-  std::vector<int> lists[3];
-  const int tz_n = (n[2] + a.zc - 1) / a.zc;
-  for (int tz = 0; tz < tz_n; ++tz)
-    for (int ty = 0; ty < a.tiles_y; ++ty)
-      for (int tx = 0; tx < a.tiles_x; ++tx) {
-        const int z0 = tz * a.zc, z1 = std::min(z0 + a.zc, n[2]), j0 = ty * e->waves, x0 = tx * 64;
-        const int m = (touches(0, x0 - 1, x0 + 64) ? 1 : 0) | (touches(1, j0 - 1, j0 + e->waves) ? 2 : 0) |
-                      (touches(2, z0 - 1, z1) ? 4 : 0);
-        lists[m == 0 ? 0 : (m == 1 ? 1 : 2)].push_back((tz * a.tiles_y + ty) * a.tiles_x + tx);
-      }
-  std::vector<int> all;
-  for (int c = 0; c < 3; ++c) {
-    e->fused_count[c] = (int)lists[c].size();
-    all.insert(all.end(), lists[c].begin(), lists[c].end());
+  // the planes between the z slabs
+  e->pass_z[0] = 0;
+  e->pass_z[1] = e->g.n[2];
+  for (int f = 0; f < 2; ++f) {
+    if (!e->pml[f][2].prof) continue;
+    const int n = e->g.n[2];
+    std::vector<float4> pr(n);
+    if ((rc = hip_check(hipMemcpy(pr.data(), e->pml[f][2].prof, n * sizeof(float4), hipMemcpyDeviceToHost),
+                        "CPML profile read")))
+      return rc;
+    int lo = 0, hi = n;
+    for (int k = 0; k < n / 2; ++k)
+      if ((int)pr[k].w >= 0) lo = k + 1;
+    for (int k = n - 1; k >= n / 2; --k)
+      if ((int)pr[k].w >= 0) hi = k;
+    e->pass_z[0] = std::max(e->pass_z[0], lo);
+    e->pass_z[1] = std::min(e->pass_z[1], hi);
   }
-  if (e->dev_tiles) (void)hipFree(e->dev_tiles);
-  e->dev_tiles = nullptr;
-  int rc = hip_check(hipMalloc(&e->dev_tiles, std::max<size_t>(1, all.size()) * sizeof(int)), "hipMalloc tile lists");
-  if (!rc) rc = hip_check(hipMemcpy(e->dev_tiles, all.data(), all.size() * sizeof(int), hipMemcpyHostToDevice),
-                          "tile list upload");
-  return rc;
+  if (!e->dev_pass) rc = hip_check(hipMalloc(&e->dev_pass, 2 * sizeof(lsf::PassArgs)), "hipMalloc pass arguments");
+  if (rc) return rc;
+  const lsf::PassArgs f[2] = {pass_args(e, 0), pass_args(e, 1)};
+  e->pass_nb = f[0].tiles_p * ((e->g.n[2] + f[0].zc - 1) / f[0].zc);
+  return hip_check(hipMemcpy(e->dev_pass, f, sizeof f, hipMemcpyHostToDevice), "pass argument upload");
 }
 
 // Upload the engine's kernel arguments (and its sub-engines') when its configuration changed. Not called
@@ -391,33 +406,24 @@ int sync_args(lsf_engine* e) {
     e->nb[f] = h[f].nb;
     e->nbp[f] = h[f].nbp;
   }
-  e->use_fused = fused_eligible(e);
-  if (e->use_fused) {
-    if (!e->dev_fused) rc = hip_check(hipMalloc(&e->dev_fused, 2 * sizeof(lsf::FusedArgs)), "hipMalloc fused arguments");
-    if (rc) return rc;
-    const lsf::FusedArgs f[2] = {fused_args(e, 0), fused_args(e, 1)};
-    rc = hip_check(hipMemcpy(e->dev_fused, f, sizeof f, hipMemcpyHostToDevice), "fused argument upload");
-    if (rc) return rc;
-    rc = fused_tiles(e, f[0]);
-    if (rc) return rc;
-  }
+  e->use_pass = pass_eligible(e);
+  if (e->use_pass && (rc = sync_pass(e, h[0]))) return rc;
   e->dirty = false;
   return LSF_OK;
 }
 
-void launch_fused_step(lsf_engine* e, hipStream_t s) {
-  lsf::FusedLaunch L{};
-  L.args = e->dev_fused + e->parity;
-  L.tiles[0] = e->dev_tiles;
-  L.tiles[1] = e->dev_tiles + e->fused_count[0];
-  L.tiles[2] = e->dev_tiles + e->fused_count[0] + e->fused_count[1];
-  for (int c = 0; c < 3; ++c) L.count[c] = e->fused_count[c];
-  L.waves = e->waves;
+// One step from buffer set `set` to the other one.
+void launch_pass_step(lsf_engine* e, int set, hipStream_t s) {
+  lsf::PassLaunch L{};
+  L.args = e->dev_pass + set;
+  L.sc = lsf::Sched{nullptr, nullptr, e->pass_nb, (e->pass_nb + 7) / 8 * 8, set ? e->rev_e : 0};
   L.mat = e->mid ? 1 : 0;
   L.np = pole_regs(e);
-  lsf::launch_fused(L, s);
+  for (int f = 0; f < 2; ++f)
+    for (int ax = 0; ax < 3; ++ax) L.kappa |= e->pml[f][ax].prof && e->pml[f][ax].has_k;
+  lsf::launch_pass(L, s);
   e->launched = true;
-  set_parity(e, e->parity ^ 1);
+  use_set(e, set ^ 1);
 }
 
 lsf::KLaunch own_launch(lsf_engine* e, int field) {
@@ -522,7 +528,9 @@ void run_op(lsf_engine* e, const Op& o, hipStream_t s) {
       break;
     case OP_TAPE: {
       lsf::TapeJob J{o.n, o.target, (const float*)e->H, e->g.n[0], e->g.n[1], e->g.N,
-                     {e->g.s[0], e->g.s[1], e->g.s[2]}, o.out, o.n_slots, o.base, (const long long*)e->counter};
+                     {e->g.s[0], e->g.s[1], e->g.s[2]}, o.out, o.n_slots, o.base,
+                     // the step's index: counter[0] before the E update advances it, counter[1] after
+                     (const long long*)e->counter + (e->passing ? 1 : 0)};
       if (o.n > 0) hipLaunchKernelGGL(lsf::k_tape, dim3(nblk(o.n, 256)), dim3(256), 0, s, J);
       break;
     }
@@ -575,18 +583,29 @@ void run_phase(lsf_engine* e, int phase, hipStream_t s) {
   }
 }
 
-void one_step(lsf_engine* e, hipStream_t s) {
-  if (e->use_fused) {
-    launch_fused_step(e, s);
+// Two steps as two single passes, there and back.
+void two_passes(lsf_engine* e, hipStream_t s) {
+  for (int set = 0; set < 2; ++set) {
+    launch_pass_step(e, set, s);
+    e->passing = true;  // the tape: H^{n+1/2} of the step just made
+    run_phase(e, LSF_PH_ADVANCE_H, s);
+    e->passing = false;
     for (int ph = LSF_PH_OFFDIAG; ph <= LSF_PH_ADVANCE_E; ++ph) run_phase(e, ph, s);
-    return;
   }
+}
+
+void one_step(lsf_engine* e, hipStream_t s) {
   run_phase(e, LSF_PH_BEFORE_H, s);
   launch_h(e, s);
   run_phase(e, LSF_PH_CORRECT_H, s);
   run_phase(e, LSF_PH_ADVANCE_H, s);
   launch_e(e, s);
   for (int ph = LSF_PH_OFFDIAG; ph <= LSF_PH_ADVANCE_E; ++ph) run_phase(e, ph, s);
+}
+
+void run_steps(lsf_engine* e, int n, hipStream_t s) {
+  for (; e->use_pass && n >= 2; n -= 2) two_passes(e, s);
+  for (; n > 0; --n) one_step(e, s);
 }
 
 template <class S>
@@ -740,10 +759,8 @@ void lsf_destroy(lsf_engine* e) {
   if (e->partial) (void)hipFree(e->partial);
   if (e->mon_tab) (void)hipFree(e->mon_tab);
   if (e->dev_args) (void)hipFree(e->dev_args);
-  if (e->dev_fused) (void)hipFree(e->dev_fused);
-  if (e->dev_tiles) (void)hipFree(e->dev_tiles);
-  if (e->exec2) (void)hipGraphExecDestroy(e->exec2);
-  if (e->graph2) (void)hipGraphDestroy(e->graph2);
+  if (e->dev_pass) (void)hipFree(e->dev_pass);
+  if (e->dform) (void)hipFree(e->dform);
   delete e;
 }
 
@@ -780,7 +797,7 @@ int lsf_set_pml(lsf_engine* e, int field, int axis, const void* prof, int n_slab
   for (int c = 0; c < 3; ++c)
     if (c != axis && prof && !ax.psi[c]) return fail(LSF_EINVAL, "missing psi array");
   if (field == 1)
-    for (int c = 0; c < 3; ++c) e->psiH[e->parity][axis][c] = ax.psi[c];
+    for (int c = 0; c < 3; ++c) e->psiH[0][axis][c] = ax.psi[c];
   return LSF_OK;
 }
 
@@ -1221,7 +1238,7 @@ int lsf_step(lsf_engine* e, int n, void* stream) {
   if (!e->cbd && !e->mid) return fail(LSF_ESTATE, "no material set");
   if (int rc1 = sync_args(e)) return rc1;
   hipStream_t s = (hipStream_t)stream;
-  for (int q = 0; q < n; ++q) one_step(e, s);
+  run_steps(e, n, s);
   return hip_check(hipGetLastError(), "step launch");
 }
 
@@ -1265,7 +1282,7 @@ int lsf_step_noalloc(lsf_engine* e, int n, void* stream) {
     if (o.kind == OP_SUB_H)
       return fail(LSF_EINVAL, "lsf_step_noalloc: an engine with sub-engines needs more kernel-argument scratch "
                               "than the 8 KiB it holds; use lsf_step");
-  if (fused_eligible(e))
+  if (e->asked_fused && pass_eligible(e))
     return fail(LSF_EINVAL, "lsf_step_noalloc: single-pass stepping is not supported; use lsf_step");
   const size_t need = 2 * sizeof(StepArgs);
   if (need > kNoAllocScratchBytes) return fail(LSF_EINVAL, "lsf_step_noalloc: kernel arguments exceed the scratch");
@@ -1284,7 +1301,6 @@ int lsf_step_noalloc(lsf_engine* e, int n, void* stream) {
   // stream-ordered upload: kernels of an earlier call on this stream have read the previous contents
   if (int rc = hip_check(hipMemcpyAsync(p, e->host_args, need, hipMemcpyHostToDevice, s), "argument staging"))
     return rc;
-  e->use_fused = false;
   e->args_override = (const StepArgs*)p;
   for (int q = 0; q < n; ++q) one_step(e, s);
   e->args_override = nullptr;
@@ -1298,21 +1314,30 @@ int lsf_step_timed(lsf_engine* e, int n, void* stream, double* ms) {
   if (int rc1 = sync_args(e)) return rc1;
   hipStream_t s = (hipStream_t)stream;
   std::vector<hipEvent_t> ev(4 * (size_t)n, nullptr);
-  int rc = LSF_OK;
+  int rc = LSF_OK, passes = 0;
   for (auto& x : ev)
     if ((rc = hip_check(hipEventCreate(&x), "event create"))) break;
   if (!rc) {
     for (int q = 0; q < n; ++q) {
-      run_phase(e, LSF_PH_BEFORE_H, s);
-      (void)hipEventRecord(ev[4 * q + 0], s);
-      if (!e->use_fused) launch_h(e, s);
-      (void)hipEventRecord(ev[4 * q + 1], s);
-      run_phase(e, LSF_PH_CORRECT_H, s);
-      run_phase(e, LSF_PH_ADVANCE_H, s);
-      (void)hipEventRecord(ev[4 * q + 2], s);
-      if (e->use_fused) launch_fused_step(e, s);  // the single pass is reported as the E time
-      else launch_e(e, s);
+      const bool pass = e->use_pass && (passes > 0 || n - q >= 2);  // steps go in pairs
+      if (pass) {
+        for (int x = 0; x < 3; ++x) (void)hipEventRecord(ev[4 * q + x], s);
+        launch_pass_step(e, passes, s);  // reported as the E time
+        passes ^= 1;
+      } else {
+        run_phase(e, LSF_PH_BEFORE_H, s);
+        (void)hipEventRecord(ev[4 * q + 0], s);
+        launch_h(e, s);
+        (void)hipEventRecord(ev[4 * q + 1], s);
+        run_phase(e, LSF_PH_CORRECT_H, s);
+        run_phase(e, LSF_PH_ADVANCE_H, s);
+        (void)hipEventRecord(ev[4 * q + 2], s);
+        launch_e(e, s);
+      }
       (void)hipEventRecord(ev[4 * q + 3], s);
+      e->passing = pass;
+      if (pass) run_phase(e, LSF_PH_ADVANCE_H, s);
+      e->passing = false;
       for (int ph = LSF_PH_OFFDIAG; ph <= LSF_PH_ADVANCE_E; ++ph) run_phase(e, ph, s);
     }
     rc = hip_check(hipGetLastError(), "timed step launch");
@@ -1324,7 +1349,7 @@ int lsf_step_timed(lsf_engine* e, int n, void* stream, double* ms) {
       float a = 0.f, b = 0.f;
       (void)hipEventElapsedTime(&a, ev[4 * q + 0], ev[4 * q + 1]);
       (void)hipEventElapsedTime(&b, ev[4 * q + 2], ev[4 * q + 3]);
-      th += e->use_fused ? 0.0 : a;  // no H kernel in a single pass
+      th += e->use_pass && q < n / 2 * 2 ? 0.0 : a;  // no H kernel in a single pass
       te += b;
     }
     ms[0] += th;
@@ -1348,7 +1373,7 @@ int lsf_chunk(lsf_engine* e, int n_chunks, int stride, void* stream) {
   if (int rc1 = sync_args(e)) return rc1;
   hipStream_t s = (hipStream_t)stream;
   for (int c = 0; c < n_chunks; ++c) {
-    for (int q = 0; q < stride; ++q) one_step(e, s);
+    run_steps(e, stride, s);
     sample(e, s);
   }
   return hip_check(hipGetLastError(), "chunk launch");
@@ -1360,7 +1385,7 @@ namespace {
 int capture_chunk(lsf_engine* e, int stride, hipStream_t s, hipGraph_t* graph, hipGraphExec_t* exec) {
   int rc = hip_check(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "begin capture");
   if (rc) return rc;
-  for (int q = 0; q < stride; ++q) one_step(e, s);
+  run_steps(e, stride, s);
   sample(e, s);
   hipGraph_t g = nullptr;
   rc = hip_check(hipStreamEndCapture(s, &g), "end capture");
@@ -1386,48 +1411,54 @@ int lsf_graph_capture(lsf_engine* e, int stride, void* stream) {
   if (stride < 1) return fail(LSF_EINVAL, "stride must be >= 1");
   if (int rc1 = sync_args(e)) return rc1;
   hipStream_t s = (hipStream_t)stream;
-  const int p0 = e->parity;
-  int rc = capture_chunk(e, stride, s, &e->graph, &e->exec);  // the capture advances the host parity only
-  if (!rc && e->use_fused && (stride & 1)) rc = capture_chunk(e, stride, s, &e->graph2, &e->exec2);
-  set_parity(e, p0);
-  e->graph_parity = p0;
-  e->graph_stride = stride;
-  return rc;
+  return capture_chunk(e, stride, s, &e->graph, &e->exec);
 }
 
 int lsf_graph_replay(lsf_engine* e, int n, void* stream) {
   if (valid(e)) return LSF_EINVAL;
   if (!e->exec) return fail(LSF_ESTATE, "no captured graph");
   for (int q = 0; q < n; ++q) {
-    hipGraphExec_t x = (e->exec2 && e->parity != e->graph_parity) ? e->exec2 : e->exec;
-    const int rc = hip_check(hipGraphLaunch(x, (hipStream_t)stream), "graph launch");
+    const int rc = hip_check(hipGraphLaunch(e->exec, (hipStream_t)stream), "graph launch");
     if (rc) return rc;
-    if (e->use_fused && (e->graph_stride & 1)) set_parity(e, e->parity ^ 1);
   }
   return LSF_OK;
 }
 
-int lsf_parity(lsf_engine* e) { return e ? e->parity : 0; }
+int lsf_parity(lsf_engine*) { return 0; }
 
-int lsf_set_fused(lsf_engine* e, void* E2, void* H2, void* const* psiH2) {
+int lsf_can_pair(lsf_engine* e) {
+  if (!e) return 0;
+  const bool had = e->pair_set;
+  e->pair_set = true;
+  const int ok = !pass_eligible(e) ? 0 : pass_pays(e) ? 2 : 1;
+  e->pair_set = had;
+  return ok;
+}
+
+int lsf_set_pair(lsf_engine* e, void* E2, void* H2, void* const* psiH2) {
   if (int rc0 = configurable(e)) return rc0;
   if (!E2 || !H2) return fail(LSF_EINVAL, "missing second field buffers");
   if (e->exec) return fail(LSF_ESTATE, "the engine has a captured graph; reset it first");
-  if (e->parity != 0) return fail(LSF_ESTATE, "second buffers are set before stepping");
-  e->Ebuf[1] = E2;
-  e->Hbuf[1] = H2;
   for (int ax = 0; ax < 3; ++ax) {
     for (int c = 0; c < 3; ++c) e->psiH[1][ax][c] = nullptr;
     if (!e->pml[1][ax].prof) continue;
     if (!psiH2 || !psiH2[ax]) return fail(LSF_EINVAL, "missing second H-side psi set");
-    const long long gap = psi_gap(e, 1, ax, 0);
+    const long long gap = psi_gap(e, ax);
     if (gap < 0) return fail(LSF_EINVAL, "the H-side psi arrays of an axis must be contiguous");
     const int c1 = ax == 0 ? 1 : 0, c2 = ax == 2 ? 1 : 2;
     e->psiH[1][ax][c1] = psiH2[ax];
     e->psiH[1][ax][c2] = (float*)psiH2[ax] + gap;
   }
-  e->fused_set = true;
+  e->Ebuf[1] = E2;
+  e->Hbuf[1] = H2;
+  e->pair_set = true;
   return LSF_OK;
+}
+
+int lsf_set_fused(lsf_engine* e, void* E2, void* H2, void* const* psiH2) {
+  const int rc = lsf_set_pair(e, E2, H2, psiH2);
+  if (!rc) e->asked_fused = true;
+  return rc;
 }
 
 int lsf_graph_reset(lsf_engine* e) {
@@ -1436,12 +1467,8 @@ int lsf_graph_reset(lsf_engine* e) {
   if (e->exec || e->graph) rc = hip_check(hipDeviceSynchronize(), "synchronize before graph reset");
   if (e->exec) (void)hipGraphExecDestroy(e->exec);
   if (e->graph) (void)hipGraphDestroy(e->graph);
-  if (e->exec2) (void)hipGraphExecDestroy(e->exec2);
-  if (e->graph2) (void)hipGraphDestroy(e->graph2);
   e->exec = nullptr;
   e->graph = nullptr;
-  e->exec2 = nullptr;
-  e->graph2 = nullptr;
   return rc;
 }
 

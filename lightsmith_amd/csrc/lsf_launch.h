@@ -46,18 +46,16 @@ constexpr int FLAT_CELLS = 2, FLAT_WAVES = 4;
 void launch_flat_h(const KLaunch& L, hipStream_t s);
 void launch_flat_e(const KLaunch& L, hipStream_t s);
 
-// the single-pass step (real fields, no periodic axes, one row per wavefront, 64 x cells): lsf_k_fused.hip
-struct FusedArgs;
-// The tiles are split three ways by the CPML axes they touch (their halos included): none, x only, any other;
-// each class runs its own kernel (the psi paths of absent axes compiled out) over its tile list.
-struct FusedLaunch {
-  const FusedArgs* args;  // device, one entry
-  const int* tiles[3];    // device tile lists: no CPML, x CPML only, other
-  int count[3];
-  int waves;
-  int mat, np;
+// the single-pass step (lsf_pass.h)
+struct PassArgs;
+struct PassLaunch {
+  const PassArgs* args;  // device, one entry per member
+  Sched sc;
+  int mat, np, kappa;
 };
-void launch_fused(const FusedLaunch& L, hipStream_t s);
+void launch_pass(const PassLaunch& L, hipStream_t s);
+// the D-form chunk table of an engine (n = 3 chunks of every row) from its E kernel arguments
+void launch_dform_chunks(const StepArgs& a, void* out, long long n, hipStream_t s);
 
 // adjoint kernels (real fields, no periodic axes, no D-form nodes; one tile per block): lsf_k_adj.hip
 void launch_adjoint_h(const KLaunch& L, hipStream_t s);

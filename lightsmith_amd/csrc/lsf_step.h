@@ -706,7 +706,8 @@ __device__ __forceinline__ void e_tile(const StepArgs& a, int t, const float* ta
 }
 
 // A member's tile 0 advances its step counter: counter[1] = n, counter[0] = n + 1 (engine.py:678).
-__device__ __forceinline__ void tick_counter(const StepArgs& a, int lt) {
+template <class A>
+__device__ __forceinline__ void tick_counter(const A& a, int lt) {
   if (a.tick && lt == 0 && threadIdx.x == 0) {
     long long* cnt = (long long*)as_global(a.counter);
     const long long n = cnt[0];
@@ -716,8 +717,8 @@ __device__ __forceinline__ void tick_counter(const StepArgs& a, int lt) {
 }
 
 // A member's LDS tables (indexed material, D-form media); `again`: the block held another member's before.
-template <int MAT, int WAVES, int NP>
-__device__ __forceinline__ void load_tables(const StepArgs& a, bool again, float* tab, float4* med_tab) {
+template <int MAT, int WAVES, int NP, class A>
+__device__ __forceinline__ void load_tables(const A& a, bool again, float* tab, float4* med_tab) {
   if (again) __syncthreads();  // the previous member's readers are done
   if (MAT == 1)
     for (int q = threadIdx.x; q < 256; q += 64 * WAVES) tab[q] = ((const float*)as_global(a.mtab))[q];

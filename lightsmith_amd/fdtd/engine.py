@@ -291,9 +291,9 @@ class Engine:
     tiling = (1, 4, 64, 8)
     # launch the tensor nodes' D update with the E-side table correction when their nodes are disjoint
     fuse_sparse = True
-    # default of the `fused` argument: step eligible engines (real fields, no periodic axes, one row per lane,
-    # 64-cell rows, no H-phase operations) with the single-pass kernel over a second buffer set
-    single_pass = False
+    # default of the `fused` argument: step eligible engines (real fields, no periodic axes, a one-row four-wavefront
+    # tile shape, no H-phase operations) in pairs of single passes over a second buffer set where that is faster
+    single_pass = True
 
     def __init__(self, device=None, *, shape, dx, dt: float, single: bool = True, inv_eps: np.ndarray,
                  groups=(), pml: PMLSpec | None = None, sources=(), monitors=(), dft_stride: int = 1,
@@ -332,16 +332,11 @@ class Engine:
         self._state = []  # device arrays the stepping writes (psi, pole and group state, source lines)
         self._subs = []  # sub-engines stepped inside this one
         self._held = 0  # batches stepping this engine
-        # single-pass stepping (lsf_set_fused): a second buffer set for real non-periodic grids
-        self._two_sets = (fused if fused is not None else Engine.single_pass) and not self.complex and not any(self.periodic) \
-            and self.tiling[0] == 1 and self.tiling[2] == 64 and not _sub
-        nsets = 2 if self._two_sets else 1
-        self._E_bufs = [torch.zeros(3 * self.N, dtype=self.fdt, device=self._dev) for _ in range(nsets)]
-        self._H_bufs = [torch.zeros(3 * self.N, dtype=self.fdt, device=self._dev) for _ in range(nsets)]
+        self.E_flat = torch.zeros(3 * self.N, dtype=self.fdt, device=self._dev)
+        self.H_flat = torch.zeros(3 * self.N, dtype=self.fdt, device=self._dev)
         view = lambda t: t.view(3, n2, n1, n0).permute(0, 3, 2, 1)  # noqa: E731
-        self._E_views = [view(t) for t in self._E_bufs]
-        self._H_views = [view(t) for t in self._H_bufs]
-        self._psiH_blocks = []  # (block, size): the H-side psi arrays of an axis, both sets
+        self.E, self.H = view(self.E_flat), view(self.H_flat)
+        self._psiH_size = [0, 0, 0]  # H-side psi values per axis
         self._counter = _counter if _counter is not None else torch.zeros(2, dtype=torch.int64, device=self._dev)
         self.n = self._counter[0:1]
         self.n_host = 0
@@ -359,7 +354,7 @@ class Engine:
         for a in range(3):
             kl = self.bloch[a] * (self.shape[a] - 2) * self.spacing[a] if self.periodic[a] else 0.0
             g.bloch_phase[a][0], g.bloch_phase[a][1] = np.cos(kl), np.sin(kl)
-        g.dev_E, g.dev_H, g.dev_counter = ptr(self._E_bufs[0]), ptr(self._H_bufs[0]), ptr(self._counter)
+        g.dev_E, g.dev_H, g.dev_counter = ptr(self.E_flat), ptr(self.H_flat), ptr(self._counter)
         g.tick = 0 if _sub else 1
         handle = ctypes.c_void_p()
         check(self.lib.lsf_create(ctypes.byref(g), ctypes.byref(handle)), "lsf_create")
@@ -405,9 +400,24 @@ class Engine:
             self.fused_table_tensor = not hit.size and self.lib.lsf_fuse_table_tensor(self._h) == 0
         self._graph_stream = None
         self._graphed = False
-        if self._two_sets:
-            arr = (ctypes.c_void_p * 3)(*[None if t is None else t.data_ptr() for t in self._psiH_second])
-            check(self.lib.lsf_set_fused(self._h, ptr(self._E_bufs[1]), ptr(self._H_bufs[1]), arr), "lsf_set_fused")
+        # single-pass stepping: a second set of E, H and H-side psi that the step alternates with; the state is in the
+        # first whenever the host has control, so the second is scratch (24 bytes a cell)
+        self._two_sets = False
+        can = 0 if _sub else self.lib.lsf_can_pair(self._h)  # 1: it could, 2: and it is the faster step
+        if (can == 2 and Engine.single_pass) if fused is None else (can and fused):
+            try:
+                sets = [torch.empty_like(self.E_flat), torch.empty_like(self.H_flat)] + \
+                    [torch.empty(n, dtype=self.fdt, device=self._dev) if n else None for n in self._psiH_size]
+            except torch.cuda.OutOfMemoryError:  # the two-kernel step needs no second set
+                if fused:
+                    raise
+                sets = None
+            if sets is not None:
+                self._keep += [t for t in sets if t is not None]
+                arr = (ctypes.c_void_p * 3)(*[None if t is None else t.data_ptr() for t in sets[2:]])
+                give = self.lib.lsf_set_fused if fused else self.lib.lsf_set_pair
+                check(give(self._h, ptr(sets[0]), ptr(sets[1]), arr), "lsf_set_pair")
+                self._two_sets = True
 
     def set_tiling(self, rows_per_lane: int, waves: int, x_cells: int, z_chunk: int):
         """Launch tiling of this engine's bulk kernels (lsf_set_tiling); before a graph is captured."""
@@ -417,27 +427,10 @@ class Engine:
               "lsf_set_tiling")
         self.tiling = (int(rows_per_lane), int(waves), int(x_cells), int(z_chunk))
 
-    # --- fields: the current buffer set ------------------------------------------------------
     @property
     def parity(self) -> int:
-        """Which buffer set holds the current fields (the single-pass step alternates them)."""
-        return int(self.lib.lsf_parity(self._h)) if self._two_sets else 0
-
-    @property
-    def E_flat(self) -> torch.Tensor:
-        return self._E_bufs[self.parity]
-
-    @property
-    def H_flat(self) -> torch.Tensor:
-        return self._H_bufs[self.parity]
-
-    @property
-    def E(self) -> torch.Tensor:
-        return self._E_views[self.parity]
-
-    @property
-    def H(self) -> torch.Tensor:
-        return self._H_views[self.parity]
+        """Which buffer set holds the fields: always the first (the single-pass step goes there and back)."""
+        return int(self.lib.lsf_parity(self._h))
 
     # --- helpers ---------------------------------------------------------------------------
     def native_index(self, flat) -> np.ndarray:
@@ -588,7 +581,6 @@ class Engine:
     # --- CPML (engine.py:344-418) --------------------------------------------------------------
     def _build_pml(self, spec: PMLSpec, inv_eps):
         self.pml_cells = tuple(tuple(int(v) for v in c) for c in spec.cells)
-        self._psiH_second = [None, None, None]
         self.n_psi = 0  # psi values allocated (slab extent x full extent of the other two axes)
         self.n_psi_stepped = 0  # psi values the update touches (slab extent x the component's stepped box)
         for d in range(3):
@@ -605,15 +597,10 @@ class Engine:
                 size = ns * others[0] * others[1]
                 psis = [None, None, None]
                 regions = self.RE if fld == 0 else self.RH
-                # both components of an axis in one allocation (the single-pass kernel addresses them from one
-                # base); the H side of a two-set engine holds both sets
-                if fld == 1 and self._two_sets:
-                    block = torch.zeros(4 * size, dtype=self.fdt, device=self._dev)
-                    self._keep.append(block)
-                    self._psiH_blocks.append((block, size))
-                    self._state.append(len(self._psiH_blocks) - 1)  # resolved to the current set by parity
-                else:
-                    block = self.zeros(2 * size)
+                # both components of an axis in one allocation (the second set of lsf_set_pair is laid out like it)
+                block = self.zeros(2 * size)
+                if fld == 1:
+                    self._psiH_size[d] = 2 * size
                 comps = [c for c in range(3) if c != d]
                 for c in range(3):
                     if c != d:
@@ -626,8 +613,6 @@ class Engine:
                 tprof = self.to_device(prof.astype(np.float32))
                 check(self.lib.lsf_set_pml(self._h, fld, d, ptr(tprof), ns, ptr(psis[0]), ptr(psis[1]),
                                            ptr(psis[2]), int(has_k)), "lsf_set_pml")
-                if fld == 1 and self._two_sets:
-                    self._psiH_second[d] = block[2 * size:]
 
     # --- mixed (interface) groups (engine.py:743-791) --------------------------------------------
     def _build_mixed(self, groups):
@@ -938,13 +923,7 @@ class Engine:
         state, source lines, monitor accumulators, sub-engines'), each once: a snapshot of these restores the
         run exactly."""
         out, seen = [], set()
-        par = self.parity
-        ts = [self.E_flat, self.H_flat, self._counter, self.energy]
-        for t in self._state:  # an int names an H-side psi block of a two-set engine: its current half
-            if isinstance(t, int):
-                block, size = self._psiH_blocks[t]
-                t = block[par * 2 * size:(par + 1) * 2 * size]
-            ts.append(t)
+        ts = [self.E_flat, self.H_flat, self._counter, self.energy, *self._state]
         for m in self.monitors:
             ts += [getattr(m, "acc_e", None), getattr(m, "acc_h", None)]
         for m in self.time_monitors:
