@@ -83,6 +83,7 @@ struct Op {
   // tensor op then skips its own D launch (lsf_fuse_table_tensor)
   int fuse_tensor = -1;
   int d_fused = 0;
+  int in_bulk = 0;  // a bulk kernel that takes corrections makes this one (plan_corr)
 };
 
 struct Monitor {
@@ -142,6 +143,17 @@ struct lsf_engine {
   int flat[2] = {0, 0};                // planes per tile of the flat E [0] and H [1] kernels; 0: the row kernels
   int nb[2] = {0, 0}, nbp[2] = {0, 0};  // tiles of the E [0] and H [1] launches (and padded to a multiple of 8)
   bool dirty = true;                   // dev_args out of date
+  // corrections made by the bulk kernels (library scratch: their row tables and the step word)
+  lsf::Corrs corr[2]{};                // [E, H]
+  std::vector<int*> corr_rows;
+  long long* step_word = nullptr;
+  bool corr_planned = false;
+  // the launches of an engine and the sub-engines that join it (joins), E [0] and H [1]; library scratch
+  bool joined = false;
+  const lsf::StepArgs* join_args[2] = {nullptr, nullptr};
+  lsf::Sched join_sc[2]{};
+  std::vector<void*> join_mem;
+  bool corr_off = false;               // stepping without them (lsf_step_noalloc)
   bool launched = false;               // kernels may be reading dev_args
   int held = 0;                        // batches holding this engine (its configuration is then frozen)
   int adjoint = 0;                     // steps the adjoint (transposed, time-reversed) update
@@ -174,10 +186,12 @@ int pole_regs(const lsf_engine* e) { return e->n_ade > 0 ? e->max_poles : 0; }
 
 bool any_periodic(const lsf_engine* e) { return e->g.per[0] || e->g.per[1] || e->g.per[2]; }
 
+bool takes_flat(const Tiling& t) { return t.ry == 1 && t.waves == lsf::FLAT_WAVES; }
+
 // Engines with a periodic axis take the flat kernels for the one-row, four-wavefront tile shapes (what the drivers
 // and the default pick), except for the E update of D-form nodes.
 bool flat_kernel(const lsf_engine* e, int field, const Tiling& t) {
-  return any_periodic(e) && !e->adjoint && t.ry == 1 && t.waves == lsf::FLAT_WAVES && (field == 1 || pole_regs(e) == 0);
+  return any_periodic(e) && !e->adjoint && takes_flat(t) && (field == 1 || pole_regs(e) == 0);
 }
 
 int flat_lpr(const lsf_engine* e) { return (e->g.n[0] + lsf::FLAT_CELLS - 1) / lsf::FLAT_CELLS; }
@@ -216,6 +230,7 @@ StepArgs make_args(const lsf_engine* e, int field, const Tiling& t, int flat) {
   a.n_media_floats = e->n_ade > 0 ? e->n_media * (2 + 3 * e->max_poles) : 0;
   a.counter = e->counter;
   a.tick = e->tick;
+  if (flat && !e->corr_off) a.corr = e->corr[field];
   const int rows = t.ry * t.waves * (64 / t.xw);
   a.tiles_x = (e->g.n[0] + t.xw - 1) / t.xw;
   a.tiles_y = (e->g.n[1] + rows - 1) / rows;
@@ -265,7 +280,7 @@ long long psi_gap(const lsf_engine* e, int ax) {
 // mirror planes, no work between the H and the E update, a one-row, four-wavefront tile shape (the default and what the
 // drivers choose; another shape asks for the row kernels) and components below 4 GB (32-bit offsets).
 bool pass_eligible(const lsf_engine* e) {
-  if (!e->pair_set || e->cplx || any_periodic(e) || e->adjoint || e->ry != 1 || e->waves != lsf::PASS_WAVES ||
+  if (!e->pair_set || !e->tick || e->cplx || any_periodic(e) || e->adjoint || e->ry != 1 || e->waves != lsf::PASS_WAVES ||
       has_h_phase_ops(e))
     return false;
   for (int c = 0; c < 3; ++c) {
@@ -340,7 +355,8 @@ lsf::PassArgs pass_args(const lsf_engine* e, int set) {
   a.n_media_floats = e->n_ade > 0 ? e->n_media * (2 + 3 * e->max_poles) : 0;
   a.media = e->media;
   a.counter = e->counter;
-  a.tick = e->tick;
+  a.second = set;
+  a.corr = e->corr[0];
   const long long cells = (long long)e->g.n[0] * e->g.n[1];
   const int per_block = lsf::PASS_OWN * lsf::PASS_WAVES;
   a.tiles_p = (int)((cells + per_block - 1) / per_block);
@@ -384,11 +400,164 @@ int sync_pass(lsf_engine* e, const StepArgs& ea) {
   return hip_check(hipMemcpy(e->dev_pass, f, sizeof f, hipMemcpyHostToDevice), "pass argument upload");
 }
 
+int dev_upload(const void* src, size_t bytes, void** dst, std::vector<void*>& owned) {
+  *dst = nullptr;
+  if (bytes == 0) return LSF_OK;
+  int rc = hip_check(hipMalloc(dst, bytes), "hipMalloc batch plan");
+  if (rc) return rc;
+  owned.push_back(*dst);
+  return hip_check(hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice), "batch plan upload");
+}
+
+// A work list over members with the given block counts: block -> member, member -> first block.
+int make_sched(const std::vector<int>& counts, lsf::Sched* sc, std::vector<void*>& owned) {
+  std::vector<int> inst, first;
+  for (size_t m = 0; m < counts.size(); ++m) {
+    first.push_back((int)inst.size());
+    inst.insert(inst.end(), counts[m], (int)m);
+  }
+  sc->n_tiles = (int)inst.size();
+  sc->n_pad = (sc->n_tiles + 7) / 8 * 8;
+  void *di = nullptr, *df = nullptr;
+  int rc = dev_upload(inst.data(), sizeof(int) * inst.size(), &di, owned);
+  if (!rc) rc = dev_upload(first.data(), sizeof(int) * first.size(), &df, owned);
+  sc->inst_of = (const int*)di;
+  sc->first = (const int*)df;
+  return rc;
+}
+
+// Give the leading gathers and modal sources that follow a field's update to the bulk kernel (Corr). An operation stays a
+// launch, and those behind it with it, where its rows repeat a node or name one that does not step, read what the bulk
+// kernel writes, or lie so thin in their box that the table would outgrow them (more than 16 entries a row), and past
+// MAX_CORR; so do all behind an off-diagonal gather.
+std::vector<Op*> in_order(lsf_engine* e, int field) {  // what runs after a field's update
+  std::vector<Op*> v;
+  for (int ph = field ? LSF_PH_CORRECT_H : LSF_PH_OFFDIAG; ph <= (field ? LSF_PH_ADVANCE_H : LSF_PH_ADVANCE_E); ++ph)
+    for (Op& o : e->ops)
+      if (o.phase == ph && o.kind != OP_VIEW) v.push_back(&o);
+  return v;
+}
+
+int plan_corr(lsf_engine* e) {
+  if (e->corr_planned) return LSF_OK;
+  int rc = LSF_OK;
+  if (!e->corr_rows.empty()) {
+    if ((rc = hip_check(hipDeviceSynchronize(), "synchronize before planning corrections"))) return rc;
+    for (int* p : e->corr_rows) (void)hipFree(p);
+    e->corr_rows.clear();
+  }
+  if (!e->step_word && (rc = hip_check(hipMalloc(&e->step_word, sizeof(long long)), "hipMalloc step word"))) return rc;
+  const int* n = e->g.n;
+  const bool pass = pass_eligible(e);
+  for (Op& o : e->ops) o.in_bulk = 0;
+  for (int f = 0; f < 2; ++f) {
+    lsf::Corrs& cs = e->corr[f];
+    cs = lsf::Corrs{};
+    cs.step = e->step_word;
+    cs.z[0] = n[2];
+    if (!pass && !any_periodic(e)) continue;  // the row and the adjoint kernels make none
+    for (Op* po : in_order(e, f)) {
+      Op& o = *po;
+      if ((o.kind != OP_GATHER && o.kind != OP_MODAL) || o.field != f || o.phase == LSF_PH_OFFDIAG || cs.n == lsf::MAX_CORR ||
+          o.n >= (1ll << 30))
+        break;
+      if (o.n <= 0) continue;
+      if (o.kind == OP_GATHER) {
+        const char* mine = (const char*)(f ? e->H : e->E);
+        const char* src = (const char*)(o.src ? o.src : e->H);
+        const size_t size = (size_t)(3 * e->g.N) * (e->cplx ? 8 : 4);
+        if (pass || (src >= mine && src < mine + size)) break;
+      }
+      std::vector<long long> t(o.n);
+      if ((rc = hip_check(hipMemcpy(t.data(), o.target, sizeof(long long) * o.n, hipMemcpyDeviceToHost), "correction targets")))
+        return rc;
+      int lo[3] = {n[0], n[1], n[2]}, hi[3] = {-1, -1, -1};
+      auto split = [&](long long x, int& c, int (&p)[3]) {
+        c = (int)(x / e->g.N);
+        x -= c * e->g.N;
+        p[0] = (int)(x % n[0]);
+        p[1] = (int)(x / n[0] % n[1]);
+        p[2] = (int)(x / n[0] / n[1]);
+      };
+      bool ok = true;
+      for (long long r = 0; r < o.n && ok; ++r) {
+        int c, p[3];
+        ok = t[r] >= 0 && t[r] < 3 * e->g.N;
+        if (!ok) break;
+        split(t[r], c, p);
+        const auto& box = f ? e->g.rH[c] : e->g.rE[c];
+        for (int ax = 0; ax < 3; ++ax) {
+          ok = ok && p[ax] >= box[ax][0] && p[ax] < box[ax][1];
+          lo[ax] = std::min(lo[ax], p[ax]);
+          hi[ax] = std::max(hi[ax], p[ax] + 1);
+        }
+      }
+      if (!ok) break;
+      const long long vol = (long long)(hi[0] - lo[0]) * (hi[1] - lo[1]) * (hi[2] - lo[2]);
+      if (3 * vol > 16 * o.n + 4096 || 3 * vol >= (1ll << 31)) break;
+      std::vector<int> row(3 * vol, -1);
+      for (long long r = 0; r < o.n && ok; ++r) {
+        int c, p[3];
+        split(t[r], c, p);
+        int& x = row[((c * (long long)(hi[2] - lo[2]) + p[2] - lo[2]) * (hi[1] - lo[1]) + p[1] - lo[1]) * (hi[0] - lo[0]) + p[0] - lo[0]];
+        ok = x < 0;
+        x = (int)r;
+      }
+      if (!ok) break;
+      int* d = nullptr;
+      if ((rc = hip_check(hipMalloc(&d, sizeof(int) * row.size()), "hipMalloc correction rows"))) return rc;
+      e->corr_rows.push_back(d);
+      if ((rc = hip_check(hipMemcpy(d, row.data(), sizeof(int) * row.size(), hipMemcpyHostToDevice), "correction rows"))) return rc;
+      lsf::Corr& q = cs.c[cs.n++];
+      q.gather = o.kind == OP_GATHER;
+      q.width = o.width;
+      for (int ax = 0; ax < 3; ++ax) {
+        q.lo[ax] = lo[ax];
+        q.n[ax] = hi[ax] - lo[ax];
+      }
+      q.row = d;
+      q.w = o.w;
+      q.src = o.src ? o.src : e->H;
+      q.sidx = o.sidx;
+      q.table = o.table;
+      q.table_len = o.table_len;
+      q.scale = o.scale;
+      cs.z[0] = std::min(cs.z[0], lo[2]);
+      cs.z[1] = std::max(cs.z[1], hi[2]);
+      o.in_bulk = 1;
+    }
+  }
+  e->corr_planned = true;
+  return LSF_OK;
+}
+
+// Whether a sub-engine's bulk updates can run inside its engine's launches (under tiling t): flat kernels on both sides, no
+// launch of its own left, and nothing between the engine's update and its own but corrections that the engine's kernel
+// makes without reading what the sub-engine's writes. A Bloch plane source's 3 x 3 column, whose H and E launches took
+// 5 us a step each beside the engine's 17.
+bool joins(lsf_engine* e, lsf_engine* sub, const Tiling& t) {
+  for (int f = 0; f < 2; ++f) {
+    if (!flat_kernel(e, f, t) || !flat_kernel(sub, f, t)) return false;
+    const char* w = (const char*)(f ? sub->H : sub->E);
+    const size_t size = (size_t)(3 * sub->g.N) * (sub->cplx ? 8 : 4);
+    for (const Op* o : in_order(e, f)) {
+      if (o->sub == sub) break;
+      if (o->sub ? !joins(e, o->sub, t) : !o->in_bulk) return false;
+      const char* src = (const char*)o->src;
+      if (o->kind == OP_GATHER && src >= w && src < w + size) return false;
+    }
+  }
+  for (const Op& o : sub->ops)
+    if (o.sub || !o.in_bulk) return false;
+  return true;
+}
+
 // Upload the engine's kernel arguments (and its sub-engines') when its configuration changed. Not called
 // during graph capture.
 int sync_args(lsf_engine* e) {
   for (const Op& o : e->ops)
     if (o.kind == OP_SUB_H) {
+      if (o.sub->dirty) e->dirty = true;
       const int rc = sync_args(o.sub);
       if (rc) return rc;
     }
@@ -396,6 +565,7 @@ int sync_args(lsf_engine* e) {
   int rc = LSF_OK;
   if (!e->dev_args) rc = hip_check(hipMalloc(&e->dev_args, 2 * sizeof(StepArgs)), "hipMalloc kernel arguments");
   else if (e->launched) rc = hip_check(hipDeviceSynchronize(), "synchronize before an argument update");
+  if (!rc) rc = plan_corr(e);
   if (rc) return rc;
   const Tiling t = own_tiling(e);
   for (int f = 0; f < 2; ++f) e->flat[f] = flat_kernel(e, f, t) ? flat_planes(&e, 1) : 0;
@@ -406,6 +576,28 @@ int sync_args(lsf_engine* e) {
     e->nb[f] = h[f].nb;
     e->nbp[f] = h[f].nbp;
   }
+  for (void* p : e->join_mem) (void)hipFree(p);
+  e->join_mem.clear();
+  std::vector<lsf_engine*> mem{e};
+  for (Op& o : e->ops) {
+    if (o.kind != OP_SUB_H && o.kind != OP_SUB_E) continue;
+    const lsf_engine* q = o.sub;
+    o.in_bulk = q->cplx == e->cplx && !q->mid == !e->mid && joins(e, o.sub, t) && joins(e, o.sub, own_tiling(q));
+    if (o.in_bulk && o.kind == OP_SUB_H) mem.push_back(o.sub);
+  }
+  for (int f = 0; f < 2 && mem.size() > 1; ++f) {
+    std::vector<StepArgs> args;
+    std::vector<int> counts;
+    for (lsf_engine* q : mem) {
+      args.push_back(q == e ? h[f] : make_args(q, f, own_tiling(q), q->flat[f]));
+      counts.push_back(args.back().nb);
+    }
+    void* d = nullptr;
+    if ((rc = dev_upload(args.data(), sizeof(StepArgs) * args.size(), &d, e->join_mem))) return rc;
+    if ((rc = make_sched(counts, &e->join_sc[f], e->join_mem))) return rc;
+    e->join_args[f] = (const StepArgs*)d;
+  }
+  e->joined = mem.size() > 1;
   e->use_pass = pass_eligible(e);
   if (e->use_pass && (rc = sync_pass(e, h[0]))) return rc;
   e->dirty = false;
@@ -439,6 +631,11 @@ lsf::KLaunch own_launch(lsf_engine* e, int field) {
   L.mat = e->mid ? 1 : 0;
   L.np = pole_regs(e);
   L.flat = e->flat[field] > 0;
+  if (e->joined) {
+    L.args = e->join_args[field];
+    L.sc = e->join_sc[field];
+    L.grid = L.sc.n_pad;
+  }
   return L;
 }
 
@@ -460,10 +657,22 @@ inline unsigned nblk(long long n, int bs) { return (unsigned)((n + bs - 1) / bs)
 
 void run_phase(lsf_engine* e, int phase, hipStream_t s);
 
+// What a gather reads: null is the engine's own H; its own E or H, however named, is the current set's.
+const void* gather_src(const lsf_engine* e, const Op& o) {
+  if (!o.src) return e->H;
+  const size_t size = (size_t)(3 * e->g.N) * (e->cplx ? 8 : 4);
+  for (int f = 0; f < 2; ++f) {
+    const char* own = (const char*)(f ? e->Hbuf[0] : e->Ebuf[0]);
+    const char* src = (const char*)o.src;
+    if (src >= own && src < own + size) return (const char*)(f ? e->H : e->E) + (src - own);
+  }
+  return o.src;
+}
+
 template <class T>
 lsf::GatherJob<T> gather_job(lsf_engine* e, const Op& o) {
   T* F = (T*)(o.field == 0 ? e->E : e->H);
-  const T* src = o.src ? (const T*)o.src : (const T*)e->H;  // null: the engine's own (current) H
+  const T* src = (const T*)gather_src(e, o);
   return lsf::GatherJob<T>{o.n, o.width, o.target, F, src, o.sidx, (const T*)o.w, o.scale};
 }
 
@@ -573,11 +782,15 @@ void run_op(lsf_engine* e, const Op& o, hipStream_t s) {
   }
 }
 
+// The bulk kernel of the field just launched made its planned corrections (and its joined sub-engines' update): a single
+// pass, or a flat kernel.
+bool made(const lsf_engine* e, int field) { return !e->corr_off && (e->passing || e->flat[field] > 0); }
+
 // A table view's only readers are monitors, which read it when they sample: it is evaluated then (run_views), with
 // the step counters of its phase, which are the same then.
 void run_phase(lsf_engine* e, int phase, hipStream_t s) {
   for (const Op& o : e->ops) {
-    if (o.phase != phase || o.kind == OP_VIEW) continue;
+    if (o.phase != phase || o.kind == OP_VIEW || (o.in_bulk && made(e, o.field))) continue;
     if (e->cplx) run_op<c32>(e, o, s);
     else run_op<float>(e, o, s);
   }
@@ -589,8 +802,8 @@ void two_passes(lsf_engine* e, hipStream_t s) {
     launch_pass_step(e, set, s);
     e->passing = true;  // the tape: H^{n+1/2} of the step just made
     run_phase(e, LSF_PH_ADVANCE_H, s);
-    e->passing = false;
     for (int ph = LSF_PH_OFFDIAG; ph <= LSF_PH_ADVANCE_E; ++ph) run_phase(e, ph, s);
+    e->passing = false;
   }
 }
 
@@ -681,6 +894,7 @@ int configurable(lsf_engine* e) {
   if (!e) return fail(LSF_EINVAL, "null engine handle");
   if (e->held) return fail(LSF_ESTATE, "the engine is held by a batch; destroy the batch before changing it");
   e->dirty = true;
+  e->corr_planned = false;
   return LSF_OK;
 }
 
@@ -760,6 +974,9 @@ void lsf_destroy(lsf_engine* e) {
   if (e->mon_tab) (void)hipFree(e->mon_tab);
   if (e->dev_args) (void)hipFree(e->dev_args);
   if (e->dev_pass) (void)hipFree(e->dev_pass);
+  for (int* p : e->corr_rows) (void)hipFree(p);
+  for (void* p : e->join_mem) (void)hipFree(p);
+  if (e->step_word) (void)hipFree(e->step_word);
   if (e->dform) (void)hipFree(e->dform);
   delete e;
 }
@@ -1290,6 +1507,7 @@ int lsf_step_noalloc(lsf_engine* e, int n, void* stream) {
   if (int rc = scratch_address(&p)) return rc;
   hipStream_t s = (hipStream_t)stream;
   const Tiling t = own_tiling(e);
+  e->corr_off = true;  // their tables are allocations
   for (int f = 0; f < 2; ++f) {
     e->flat[f] = flat_kernel(e, f, t) ? flat_planes(&e, 1) : 0;
     e->host_args[f] = make_args(e, f, t, e->flat[f]);
@@ -1299,11 +1517,12 @@ int lsf_step_noalloc(lsf_engine* e, int n, void* stream) {
     e->nbp[f] = e->host_args[f].nbp;
   }
   // stream-ordered upload: kernels of an earlier call on this stream have read the previous contents
-  if (int rc = hip_check(hipMemcpyAsync(p, e->host_args, need, hipMemcpyHostToDevice, s), "argument staging"))
-    return rc;
+  const int rc = hip_check(hipMemcpyAsync(p, e->host_args, need, hipMemcpyHostToDevice, s), "argument staging");
   e->args_override = (const StepArgs*)p;
-  for (int q = 0; q < n; ++q) one_step(e, s);
+  for (int q = 0; !rc && q < n; ++q) one_step(e, s);
   e->args_override = nullptr;
+  e->corr_off = false;
+  if (rc) return rc;
   return hip_check(hipGetLastError(), "step launch");
 }
 
@@ -1337,8 +1556,8 @@ int lsf_step_timed(lsf_engine* e, int n, void* stream, double* ms) {
       (void)hipEventRecord(ev[4 * q + 3], s);
       e->passing = pass;
       if (pass) run_phase(e, LSF_PH_ADVANCE_H, s);
-      e->passing = false;
       for (int ph = LSF_PH_OFFDIAG; ph <= LSF_PH_ADVANCE_E; ++ph) run_phase(e, ph, s);
+      e->passing = false;
     }
     rc = hip_check(hipGetLastError(), "timed step launch");
   }
@@ -1538,39 +1757,17 @@ struct lsf_batch {
 
 namespace {
 
-int dev_upload(const void* src, size_t bytes, void** dst, std::vector<void*>& owned) {
-  *dst = nullptr;
-  if (bytes == 0) return LSF_OK;
-  int rc = hip_check(hipMalloc(dst, bytes), "hipMalloc batch plan");
-  if (rc) return rc;
-  owned.push_back(*dst);
-  return hip_check(hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice), "batch plan upload");
-}
-
-// A work list over members with the given block counts: block -> member, member -> first block.
-int make_sched(const std::vector<int>& counts, lsf::Sched* sc, std::vector<void*>& owned) {
-  std::vector<int> inst, first;
-  for (size_t m = 0; m < counts.size(); ++m) {
-    first.push_back((int)inst.size());
-    inst.insert(inst.end(), counts[m], (int)m);
-  }
-  sc->n_tiles = (int)inst.size();
-  sc->n_pad = (sc->n_tiles + 7) / 8 * 8;
-  void *di = nullptr, *df = nullptr;
-  int rc = dev_upload(inst.data(), sizeof(int) * inst.size(), &di, owned);
-  if (!rc) rc = dev_upload(first.data(), sizeof(int) * first.size(), &df, owned);
-  sc->inst_of = (const int*)di;
-  sc->first = (const int*)df;
-  return rc;
-}
-
 // Bulk-kernel groups of a level under tiling t: members sharing a kernel instantiation share a launch.
 int build_groups(Level& L, const Tiling& t, int grid_blocks, std::vector<void*>& owned) {
   L.hg.clear();
   L.eg.clear();
+  std::vector<lsf_engine*> mem = L.mem;
+  for (lsf_engine* e : L.mem)
+    for (const Op& o : e->ops)
+      if (o.kind == OP_SUB_H && joins(e, o.sub, t)) mem.push_back(o.sub);
   for (int field = 0; field < 2; ++field) {
     std::vector<KGroup>& groups = field ? L.hg : L.eg;
-    for (lsf_engine* e : L.mem) {
+    for (lsf_engine* e : mem) {
       KGroup key;
       key.cplx = e->cplx ? 1 : 0;
       key.per = any_periodic(e) ? 1 : 0;
@@ -1711,6 +1908,7 @@ int build_level(Level& L, const Tiling& t, int grid_blocks, bool sample, std::ve
       size_t q = 0;
       for (const Op& o : e->ops) {
         if (o.phase != ph || o.kind == OP_VIEW) continue;  // views run when the batch samples
+        if (o.sub ? joins(e, o.sub, t) : (o.in_bulk && flat_kernel(e, o.field, t))) continue;
         if (by_pos.size() <= q) by_pos.resize(q + 1);
         by_pos[q++].push_back({e, o});
       }
@@ -1804,6 +2002,13 @@ void batch_step(lsf_batch* b, hipStream_t s) {
   level_e(b->root, s);
 }
 
+int plan_all(lsf_engine* e) {
+  for (const Op& o : e->ops)
+    if (o.kind == OP_SUB_H)
+      if (int rc = plan_all(o.sub)) return rc;
+  return plan_corr(e);
+}
+
 void hold(lsf_engine* e, int d) {
   e->held += d;
   for (const Op& o : e->ops)
@@ -1835,7 +2040,10 @@ int lsf_batch_create(lsf_engine* const* members, int n, lsf_batch** out) {
   lsf_batch* b = new lsf_batch();
   b->members.assign(members, members + n);
   b->root.mem = b->members;
-  const int rc = build_level(b->root, b->tiling, b->grid_blocks, true, b->owned, b->owned_groups);
+  int rc = LSF_OK;
+  for (lsf_engine* e : b->members)
+    if (!rc) rc = plan_all(e);
+  if (!rc) rc = build_level(b->root, b->tiling, b->grid_blocks, true, b->owned, b->owned_groups);
   if (rc) {
     free_all(b->owned);
     free_all(b->owned_groups);
@@ -1866,10 +2074,15 @@ int lsf_batch_set_schedule(lsf_batch* b, int ry, int waves, int xw, int zc, int 
   if (b->exec) return fail(LSF_ESTATE, "the batch has a captured graph; reset it before rescheduling");
   int rc = hip_check(hipDeviceSynchronize(), "synchronize before rescheduling");
   if (rc) return rc;
+  const bool was = takes_flat(b->tiling);
   b->tiling = Tiling{ry, waves, xw, zc};
   b->grid_blocks = grid_blocks;
   free_all(b->owned_groups);
-  return build_groups(b->root, b->tiling, b->grid_blocks, b->owned_groups);
+  if (takes_flat(b->tiling) == was) return build_groups(b->root, b->tiling, b->grid_blocks, b->owned_groups);
+  free_all(b->owned);  // the kernels that make corrections come or go, and those operations' launches with them
+  b->root = Level{};
+  b->root.mem = b->members;
+  return build_level(b->root, b->tiling, b->grid_blocks, true, b->owned, b->owned_groups);
 }
 
 int lsf_batch_tiles(lsf_batch* b, int64_t* n_tiles) {

@@ -18,6 +18,53 @@
 #include "lsf_step.h"
 
 namespace lsf {
+
+// Source corrections of the cells a lane has just stored: V cells from (i, j) of the planes [z0, z1), element e on only
+// if e >= sh. The launch this replaces costs 4.5-4.9 us a step whatever its size; here a tile outside the boxes' planes
+// pays a compare. It runs after the tile's march, on the lane's own stored values: inside the march it cost the loops
+// registers (25 more scalar spills, 5 % of a Bloch cell's step). The row kernels leave their corrections to launches: even
+// at their end this slows the E kernel of 4-pole nodes from 143 to 204 us (4 boxes of 96^3). Rows are added in launch
+// order, each sum from zero, as the launches add them: the fields are the same bits.
+template <class T, int V>
+__device__ __forceinline__ void correct(const Corrs& s, const long long* step_at, long long ahead, T* F, const Grid& g,
+                                        bool own, int i, int j, int sh, int z0, int z1) {
+  z0 = max(z0, s.z[0]);
+  z1 = min(z1, s.z[1]);
+  if (s.n == 0 || z0 >= z1) return;
+  const long long step = *(const long long*)as_global(step_at) + ahead;
+  for (int q = 0; q < s.n; ++q) {
+    const Corr& o = s.c[q];
+    if (!o.gather && (step < 0 || step >= o.table_len)) continue;
+    const int n0 = o.n[0], n1 = o.n[1], n2 = o.n[2], dj = j - o.lo[1];
+    if (!own || dj < 0 || dj >= n1) continue;
+    for (int k = max(z0, o.lo[2]); k < min(z1, o.lo[2] + n2); ++k)
+      for (int e = sh; e < V; ++e) {
+        const int di = i + e - o.lo[0];
+        if (di < 0 || di >= n0) continue;
+        for (int c = 0; c < 3; ++c) {
+          const int r = ((const int*)as_global(o.row))[((c * n2 + k - o.lo[2]) * n1 + dj) * n0 + di];
+          if (r < 0) continue;
+          const T* w = (const T*)as_global((const T*)o.w) + (long long)r * o.width;
+          T acc = zero<T>();
+          if (o.gather) {
+            const long long* sidx = (const long long*)as_global(o.sidx) + (long long)r * o.width;
+            for (int p = 0; p < o.width; ++p) acc = add(acc, mul(w[p], ((const T*)as_global((const T*)o.src))[sidx[p]]));
+          } else {
+            const float* tab = (const float*)as_global(o.table) + step * o.width;
+            for (int p = 0; p < o.width; ++p) acc = add(acc, scl(tab[p], w[p]));
+          }
+          T* f = (T*)as_global(F) + (long long)c * g.N + cidx(g, i + e, j, k);
+          *f = add(*f, o.scale ? scl(((const float*)as_global(o.scale))[r], acc) : acc);
+        }
+      }
+  }
+}
+
+// The step's index where the E kernel may read it: the counter advances while that kernel runs.
+__device__ __forceinline__ void note_step(const StepArgs& a, int lt) {
+  if (lt == 0 && threadIdx.x == 0 && a.corr.step) *(long long*)as_global(a.corr.step) = *(const long long*)as_global(a.counter);
+}
+
 namespace flat {
 
 // V values of the field type from base + a 32-bit byte offset (global memory, 4-byte aligned)
@@ -372,6 +419,7 @@ __device__ __forceinline__ void h_tile(const StepArgs& a, int t) {
       cz[e] = nz_[e];
     }
   }
+  correct<T, V>(a.corr, a.counter, 0, (T*)a.H, g, q.act, q.i0, q.j, q.sh, z0, z1);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -602,6 +650,7 @@ __device__ __forceinline__ void e_tile(const StepArgs& a, int t, const float* ta
       py_[e] = hy[e];
     }
   }
+  correct<T, V>(a.corr, a.corr.step, 0, (T*)a.E, g, q.act, q.i0, q.j, q.sh, z0, z1);
 }
 
 }  // namespace flat
@@ -613,6 +662,7 @@ __global__ void __launch_bounds__(64 * WAVES) k_flat_h(const StepArgs* __restric
     if (t < sc.n_tiles) {
       int m, lt;
       member_of(sc, t, m, lt);
+      note_step(args[m], lt);
       flat::h_tile<T, V, WAVES>(args[m], lt);
     }
     if (!LOOP) break;

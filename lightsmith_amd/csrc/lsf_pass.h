@@ -57,8 +57,9 @@ struct PassArgs {
   int nchunk, media_stride, n_media_floats;
   const float* media;
   long long* counter;
-  int tick;
   int tiles_p, zc;            // tiles per plane, planes per tile
+  int second;                 // the second pass of a pair
+  Corrs corr;                 // source corrections of E
 };
 
 constexpr int PASS_WAVES = 4, PASS_OWN = 62;
@@ -534,6 +535,23 @@ __device__ __forceinline__ void tile(const PassArgs& a, int t, const float* tab,
     o1 += plane;
     o2 += plane;
   }
+  correct<float, 1>(a.corr, a.second ? a.corr.step : a.counter, a.second, a.E_out, g, own, i, j, 0, z0, z1);
+}
+
+// The pair's passes advance the step counter: counter[1] = n after each, counter[0] = n + 1 after the second only (the
+// operations that follow a pass read counter[1]). No pass writes a word that its blocks may still read: the first reads
+// counter[0] and writes counter[1] and its copy of n, the second reads the copy.
+__device__ __forceinline__ void tick_pair(const PassArgs& a, int lt) {
+  if (lt != 0 || threadIdx.x != 0) return;
+  long long* cnt = (long long*)as_global(a.counter);
+  long long* step = (long long*)as_global(a.corr.step);
+  if (a.second) {
+    const long long n = *step + 1;
+    cnt[1] = n;
+    cnt[0] = n + 1;
+  } else {
+    cnt[1] = *step = cnt[0];
+  }
 }
 
 }  // namespace pass
@@ -548,7 +566,7 @@ __global__ void __launch_bounds__(64 * PASS_WAVES) k_pass(const PassArgs* __rest
   int m, lt;
   member_of(sc, t, m, lt);
   const PassArgs& a = args[m];
-  tick_counter(a, lt);
+  pass::tick_pair(a, lt);
   if (MAT == 1 || NP > 0) load_tables<MAT, PASS_WAVES, NP>(a, false, tab, med_tab);
   pass::tile<MAT, NP, KAP>(a, lt, tab, med_tab, nodes + (NP > 0 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0));
 }

@@ -25,6 +25,29 @@ struct PmlAx {
   int has_k;           // kappa_max > 1 somewhere on this axis
 };
 
+// A source correction made by the bulk kernel that updates its nodes: the rows of a gather or a modal launch
+// (lsf_sparse.h, same arithmetic), found through a table over the box of their nodes.
+struct Corr {
+  int gather;              // 1: sum_q w src[sidx]; 0: sum_q w table[step]
+  int width;               // terms per row
+  int lo[3], n[3];         // the box
+  const int* row;          // [component][n2][n1][n0]: row of the node, -1: none
+  const void* w;           // weights / mode profiles, field type
+  const void* src;
+  const long long* sidx;
+  const float* table;
+  long long table_len;
+  const float* scale;
+};
+constexpr int MAX_CORR = 3;
+
+struct Corrs {
+  Corr c[MAX_CORR];
+  int n;
+  int z[2];                // planes [z0, z1) hold all their boxes
+  long long* step;         // the step's index for the kernels that run while the counter advances
+};
+
 struct StepArgs {
   Grid g;
   void* E;
@@ -46,6 +69,7 @@ struct StepArgs {
   int tick;
   int tiles_x, tiles_y, zc, nb, nbp;
   int lpr;               // lanes per x row of the flat kernels (tiles_x: their tiles per plane)
+  Corrs corr;            // source corrections of this kernel's field
 };
 
 // The tiles of one launch: every member's tiles laid end to end.
@@ -706,8 +730,7 @@ __device__ __forceinline__ void e_tile(const StepArgs& a, int t, const float* ta
 }
 
 // A member's tile 0 advances its step counter: counter[1] = n, counter[0] = n + 1 (engine.py:678).
-template <class A>
-__device__ __forceinline__ void tick_counter(const A& a, int lt) {
+__device__ __forceinline__ void tick_counter(const StepArgs& a, int lt) {
   if (a.tick && lt == 0 && threadIdx.x == 0) {
     long long* cnt = (long long*)as_global(a.counter);
     const long long n = cnt[0];
