@@ -106,6 +106,13 @@ struct TimeMon {
   long long* pos = nullptr;
 };
 
+// Operations of one engine that touch none of each other's data; jobs: as one launch, else the one operation it holds.
+struct Stage {
+  std::vector<Op> ops;
+  const lsf::AnyJob* jobs = nullptr;  // device
+  lsf::Sched sc{};
+};
+
 }  // namespace
 
 struct lsf_engine {
@@ -153,6 +160,10 @@ struct lsf_engine {
   const lsf::StepArgs* join_args[2] = {nullptr, nullptr};
   lsf::Sched join_sc[2]{};
   std::vector<void*> join_mem;
+  // the work before the H update [0], after it [1] and after the E update [2], where some of it shares launches
+  std::vector<Stage> stages[3];
+  bool staged = false;
+  std::vector<void*> stage_mem;
   bool corr_off = false;               // stepping without them (lsf_step_noalloc)
   bool launched = false;               // kernels may be reading dev_args
   int held = 0;                        // batches holding this engine (its configuration is then frozen)
@@ -400,6 +411,55 @@ int sync_pass(lsf_engine* e, const StepArgs& ea) {
   return hip_check(hipMemcpy(e->dev_pass, f, sizeof f, hipMemcpyHostToDevice), "pass argument upload");
 }
 
+inline unsigned nblk(long long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
+
+// kinds that k_job and k_jobs run
+bool is_job(const Op& o) {
+  switch (o.kind) {
+    case OP_LINE_H: case OP_LINE_E: case OP_TAPE: case OP_ADJ_GRAD: case OP_ADJ_ADE_PRE: case OP_ADJ_ADE_POST:
+    case OP_ADJ_SRC: return true;
+    default: return false;
+  }
+}
+
+lsf::AnyJob any_job(const lsf_engine* e, const Op& o) {
+  const int slot = o.phase <= LSF_PH_ADVANCE_H ? 0 : 1;
+  const long long* counter = e->counter;
+  lsf::AnyJob J{};
+  J.rows = o.n;
+  switch (o.kind) {
+    case OP_TAPE:
+      J.kind = lsf::JOB_TAPE;
+      J.tape = lsf::TapeJob{o.n, o.target, (const float*)e->H, e->g.n[0], e->g.n[1], e->g.N,
+                            {e->g.s[0], e->g.s[1], e->g.s[2]}, o.out, o.n_slots, o.base,
+                            // the step's index: counter[0] before the E update advances it, counter[1] after
+                            counter + (e->passing ? 1 : 0)};
+      break;
+    case OP_ADJ_GRAD:
+      J.kind = lsf::JOB_GRAD;
+      J.grad = lsf::GradJob{o.n, o.target, (const float*)e->E, o.coef, o.table, o.n_slots, o.base, counter, o.n_steps, o.gacc};
+      break;
+    case OP_ADJ_ADE_PRE:
+    case OP_ADJ_ADE_POST:
+      J.kind = o.kind == OP_ADJ_ADE_PRE ? lsf::JOB_ADE_PRE : lsf::JOB_ADE_POST;
+      J.ade = lsf::AdjAdeJob{o.n, o.target, o.ade_medium, o.coef, 2 + 3 * o.maxp, o.maxp, (float*)o.state, o.out, (float*)e->E};
+      break;
+    case OP_ADJ_SRC:
+      J.kind = lsf::JOB_ADJ_SRC;
+      J.src = lsf::AdjSrcJob{o.h_side, o.width, o.m_pts, o.omega, o.dt, (const c32*)o.w, o.n, o.row_ptr, o.target,
+                             o.t2, o.scale, (float*)(o.h_side ? e->H : e->E), counter, o.n_steps, o.dft_stride};
+      break;
+    default:
+      J.kind = o.kind == OP_LINE_H ? lsf::JOB_LINE_H : lsf::JOB_LINE_E;
+      J.line = lsf::LineJob{(int)o.n, o.e1, o.h1, o.ca, o.cb, o.da, o.db, o.m_src, o.table, o.table_len, counter, slot};
+  }
+  return J;
+}
+
+// The bulk kernel of the field just launched made its planned corrections (and its joined sub-engines' update): a single
+// pass, or a flat kernel.
+bool made(const lsf_engine* e, int field) { return !e->corr_off && (e->passing || e->flat[field] > 0); }
+
 int dev_upload(const void* src, size_t bytes, void** dst, std::vector<void*>& owned) {
   *dst = nullptr;
   if (bytes == 0) return LSF_OK;
@@ -552,6 +612,92 @@ bool joins(lsf_engine* e, lsf_engine* sub, const Tiling& t) {
   return true;
 }
 
+constexpr int HALF_PHASES[3][2] = {{LSF_PH_BEFORE_H, LSF_PH_BEFORE_H}, {LSF_PH_CORRECT_H, LSF_PH_ADVANCE_H},
+                                   {LSF_PH_OFFDIAG, LSF_PH_ADVANCE_E}};
+
+// Whether two operations of an engine, of one stretch between bulk updates, touch none of each other's data. Only the kinds
+// of k_jobs are told apart: 1D lines of their own from each other and from the rest, the adjoint's H source (adds to H)
+// from its gradient (reads E) and its D-form restore (writes E), and these two where their nodes are disjoint.
+int apart(const Op& a, const Op& b, bool* yes) {
+  auto line = [](const Op& o) { return o.kind == OP_LINE_H || o.kind == OP_LINE_E; };
+  auto h_src = [](const Op& o) { return o.kind == OP_ADJ_SRC && o.h_side; };
+  auto e_side = [](const Op& o) { return o.kind == OP_ADJ_GRAD || o.kind == OP_ADJ_ADE_POST; };
+  *yes = false;
+  if (!is_job(a) || !is_job(b)) return LSF_OK;
+  if (line(a) || line(b)) {
+    *yes = !(line(a) && line(b)) || (a.kind == b.kind && a.e1 != b.e1 && a.h1 != b.h1);
+  } else if ((h_src(a) && e_side(b)) || (h_src(b) && e_side(a))) {
+    *yes = true;
+  } else if (e_side(a) && e_side(b) && a.kind != b.kind) {
+    std::vector<long long> t[2] = {std::vector<long long>(a.n), std::vector<long long>(b.n)};
+    for (int q = 0; q < 2; ++q) {
+      const Op& o = q ? b : a;
+      if (int rc = hip_check(hipMemcpy(t[q].data(), o.target, sizeof(long long) * o.n, hipMemcpyDeviceToHost), "operation nodes"))
+        return rc;
+      std::sort(t[q].begin(), t[q].end());
+    }
+    size_t i = 0, j = 0;
+    *yes = true;
+    while (i < t[0].size() && j < t[1].size() && *yes) {
+      *yes = t[0][i] != t[1][j];
+      if (t[0][i] < t[1][j]) ++i;
+      else ++j;
+    }
+  }
+  return LSF_OK;
+}
+
+// The operations of a stretch that are still launches (taken: made by a bulk kernel or a joined launch), each with the
+// earliest stage that follows every operation it is not apart from.
+template <class Taken>
+int stages_of(const lsf_engine* e, int half, Taken taken, std::vector<std::pair<int, const Op*>>& out) {
+  for (int ph = HALF_PHASES[half][0]; ph <= HALF_PHASES[half][1]; ++ph)
+    for (const Op& o : e->ops) {
+      if (o.phase != ph || o.kind == OP_VIEW || taken(o)) continue;
+      int st = 0;
+      for (const auto& p : out) {
+        bool yes = false;
+        if (p.first >= st)
+          if (int rc = apart(*p.second, o, &yes)) return rc;
+        if (p.first >= st && !yes) st = p.first + 1;
+      }
+      out.push_back({st, &o});
+    }
+  return LSF_OK;
+}
+
+int plan_stages(lsf_engine* e) {
+  for (void* p : e->stage_mem) (void)hipFree(p);
+  e->stage_mem.clear();
+  e->staged = false;
+  for (auto& v : e->stages) v.clear();
+  if (e->use_pass) return LSF_OK;  // its steps differ in what is left to launch
+  for (int half = 0; half < 3; ++half) {
+    std::vector<std::pair<int, const Op*>> at;
+    if (int rc = stages_of(e, half, [&](const Op& o) { return o.in_bulk && made(e, o.field); }, at)) return rc;
+    std::vector<Stage>& v = e->stages[half];
+    for (const auto& p : at) {
+      if ((int)v.size() <= p.first) v.resize(p.first + 1);
+      v[p.first].ops.push_back(*p.second);
+    }
+    for (Stage& g : v) {
+      if (g.ops.size() < 2) continue;
+      std::vector<lsf::AnyJob> jobs;
+      std::vector<int> counts;
+      for (const Op& o : g.ops) {
+        jobs.push_back(any_job(e, o));
+        counts.push_back((int)nblk(o.n, 256));
+      }
+      void* d = nullptr;
+      if (int rc = dev_upload(jobs.data(), sizeof(jobs[0]) * jobs.size(), &d, e->stage_mem)) return rc;
+      if (int rc = make_sched(counts, &g.sc, e->stage_mem)) return rc;
+      g.jobs = (const lsf::AnyJob*)d;
+      e->staged = true;
+    }
+  }
+  return LSF_OK;
+}
+
 // Upload the engine's kernel arguments (and its sub-engines') when its configuration changed. Not called
 // during graph capture.
 int sync_args(lsf_engine* e) {
@@ -599,6 +745,7 @@ int sync_args(lsf_engine* e) {
   }
   e->joined = mem.size() > 1;
   e->use_pass = pass_eligible(e);
+  if ((rc = plan_stages(e))) return rc;
   if (e->use_pass && (rc = sync_pass(e, h[0]))) return rc;
   e->dirty = false;
   return LSF_OK;
@@ -653,9 +800,7 @@ void launch_e(lsf_engine* e, hipStream_t s) {
   e->launched = true;
 }
 
-inline unsigned nblk(long long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
-
-void run_phase(lsf_engine* e, int phase, hipStream_t s);
+void run_half(lsf_engine* e, int half, hipStream_t s);
 
 // What a gather reads: null is the engine's own H; its own E or H, however named, is the current set's.
 const void* gather_src(const lsf_engine* e, const Op& o) {
@@ -718,51 +863,24 @@ void run_op(lsf_engine* e, const Op& o, hipStream_t s) {
       hipLaunchKernelGGL(lsf::k_table_view, dim3(1), dim3(64), 0, s, (int)o.n, o.out, o.table, o.m, o.cmax, o.base,
                          o.i0, o.u0, (const long long*)e->counter, slot);
       break;
-    case OP_LINE_H:
-      hipLaunchKernelGGL(lsf::k_line_h, dim3(1), dim3(1024), 0, s, (int)o.n, (const float*)o.e1, o.h1, o.da, o.db);
-      break;
-    case OP_LINE_E:
-      hipLaunchKernelGGL(lsf::k_line_e, dim3(1), dim3(1024), 0, s, (int)o.n, o.e1, (const float*)o.h1, o.ca, o.cb,
-                         o.m_src, o.table, o.table_len, (const long long*)e->counter, slot);
-      break;
     case OP_SUB_H:
-      run_phase(o.sub, LSF_PH_BEFORE_H, s);
+      run_half(o.sub, 0, s);
       launch_h(o.sub, s);
-      run_phase(o.sub, LSF_PH_CORRECT_H, s);
-      run_phase(o.sub, LSF_PH_ADVANCE_H, s);
+      run_half(o.sub, 1, s);
       break;
     case OP_SUB_E:
       launch_e(o.sub, s);
-      for (int ph = LSF_PH_OFFDIAG; ph <= LSF_PH_ADVANCE_E; ++ph) run_phase(o.sub, ph, s);
+      run_half(o.sub, 2, s);
       break;
-    case OP_TAPE: {
-      lsf::TapeJob J{o.n, o.target, (const float*)e->H, e->g.n[0], e->g.n[1], e->g.N,
-                     {e->g.s[0], e->g.s[1], e->g.s[2]}, o.out, o.n_slots, o.base,
-                     // the step's index: counter[0] before the E update advances it, counter[1] after
-                     (const long long*)e->counter + (e->passing ? 1 : 0)};
-      if (o.n > 0) hipLaunchKernelGGL(lsf::k_tape, dim3(nblk(o.n, 256)), dim3(256), 0, s, J);
-      break;
-    }
-    case OP_ADJ_GRAD: {
-      lsf::GradJob J{o.n, o.target, (const float*)e->E, o.coef, o.table, o.n_slots, o.base,
-                     (const long long*)e->counter, o.n_steps, o.gacc};
-      if (o.n > 0) hipLaunchKernelGGL(lsf::k_adj_grad, dim3(nblk(o.n, 256)), dim3(256), 0, s, J);
-      break;
-    }
+    case OP_LINE_H:
+    case OP_LINE_E:
+    case OP_TAPE:
+    case OP_ADJ_GRAD:
     case OP_ADJ_ADE_PRE:
-    case OP_ADJ_ADE_POST: {
-      lsf::AdjAdeJob J{o.n, o.target, o.ade_medium, o.coef, 2 + 3 * o.maxp, o.maxp, (float*)o.state, o.out, (float*)e->E};
-      if (o.n > 0) {
-        if (o.kind == OP_ADJ_ADE_PRE) hipLaunchKernelGGL(lsf::k_adj_ade_pre, dim3(nblk(o.n, 256)), dim3(256), 0, s, J);
-        else hipLaunchKernelGGL(lsf::k_adj_ade_post, dim3(nblk(o.n, 256)), dim3(256), 0, s, J);
-      }
-      break;
-    }
+    case OP_ADJ_ADE_POST:
     case OP_ADJ_SRC: {
-      lsf::AdjSrcJob J{o.h_side, o.width, o.m_pts, o.omega, o.dt, (const c32*)o.w, o.n, o.row_ptr, o.target,
-                       o.t2, o.scale, (float*)(o.h_side ? e->H : e->E), (const long long*)e->counter, o.n_steps,
-                       o.dft_stride};
-      if (o.n > 0) hipLaunchKernelGGL(lsf::k_adj_src, dim3(nblk(o.n, 256)), dim3(256), 0, s, J);
+      const lsf::AnyJob J = any_job(e, o);
+      if (J.rows > 0) hipLaunchKernelGGL(lsf::k_job, dim3(nblk(J.rows, 256)), dim3(256), 0, s, J);
       break;
     }
     case OP_TENSOR: {
@@ -782,10 +900,6 @@ void run_op(lsf_engine* e, const Op& o, hipStream_t s) {
   }
 }
 
-// The bulk kernel of the field just launched made its planned corrections (and its joined sub-engines' update): a single
-// pass, or a flat kernel.
-bool made(const lsf_engine* e, int field) { return !e->corr_off && (e->passing || e->flat[field] > 0); }
-
 // A table view's only readers are monitors, which read it when they sample: it is evaluated then (run_views), with
 // the step counters of its phase, which are the same then.
 void run_phase(lsf_engine* e, int phase, hipStream_t s) {
@@ -802,18 +916,34 @@ void two_passes(lsf_engine* e, hipStream_t s) {
     launch_pass_step(e, set, s);
     e->passing = true;  // the tape: H^{n+1/2} of the step just made
     run_phase(e, LSF_PH_ADVANCE_H, s);
-    for (int ph = LSF_PH_OFFDIAG; ph <= LSF_PH_ADVANCE_E; ++ph) run_phase(e, ph, s);
+    run_half(e, 2, s);
     e->passing = false;
   }
 }
 
+// The work of a stretch: before the H update (0), after it (1), after the E update (2).
+void run_half(lsf_engine* e, int half, hipStream_t s) {
+  if (!e->staged || e->corr_off) {
+    for (int ph = HALF_PHASES[half][0]; ph <= HALF_PHASES[half][1]; ++ph) run_phase(e, ph, s);
+    return;
+  }
+  for (const Stage& g : e->stages[half]) {
+    if (g.jobs) {
+      if (g.sc.n_tiles > 0) hipLaunchKernelGGL(lsf::k_jobs, dim3(g.sc.n_tiles), dim3(256), 0, s, g.jobs, g.sc);
+    } else if (e->cplx) {
+      for (const Op& o : g.ops) run_op<c32>(e, o, s);
+    } else {
+      for (const Op& o : g.ops) run_op<float>(e, o, s);
+    }
+  }
+}
+
 void one_step(lsf_engine* e, hipStream_t s) {
-  run_phase(e, LSF_PH_BEFORE_H, s);
+  run_half(e, 0, s);
   launch_h(e, s);
-  run_phase(e, LSF_PH_CORRECT_H, s);
-  run_phase(e, LSF_PH_ADVANCE_H, s);
+  run_half(e, 1, s);
   launch_e(e, s);
-  for (int ph = LSF_PH_OFFDIAG; ph <= LSF_PH_ADVANCE_E; ++ph) run_phase(e, ph, s);
+  run_half(e, 2, s);
 }
 
 void run_steps(lsf_engine* e, int n, hipStream_t s) {
@@ -976,6 +1106,7 @@ void lsf_destroy(lsf_engine* e) {
   if (e->dev_pass) (void)hipFree(e->dev_pass);
   for (int* p : e->corr_rows) (void)hipFree(p);
   for (void* p : e->join_mem) (void)hipFree(p);
+  for (void* p : e->stage_mem) (void)hipFree(p);
   if (e->step_word) (void)hipFree(e->step_word);
   if (e->dform) (void)hipFree(e->dform);
   delete e;
@@ -1544,19 +1675,18 @@ int lsf_step_timed(lsf_engine* e, int n, void* stream, double* ms) {
         launch_pass_step(e, passes, s);  // reported as the E time
         passes ^= 1;
       } else {
-        run_phase(e, LSF_PH_BEFORE_H, s);
+        run_half(e, 0, s);
         (void)hipEventRecord(ev[4 * q + 0], s);
         launch_h(e, s);
         (void)hipEventRecord(ev[4 * q + 1], s);
-        run_phase(e, LSF_PH_CORRECT_H, s);
-        run_phase(e, LSF_PH_ADVANCE_H, s);
+        run_half(e, 1, s);
         (void)hipEventRecord(ev[4 * q + 2], s);
         launch_e(e, s);
       }
       (void)hipEventRecord(ev[4 * q + 3], s);
       e->passing = pass;
       if (pass) run_phase(e, LSF_PH_ADVANCE_H, s);
-      for (int ph = LSF_PH_OFFDIAG; ph <= LSF_PH_ADVANCE_E; ++ph) run_phase(e, ph, s);
+      run_half(e, 2, s);
       e->passing = false;
     }
     rc = hip_check(hipGetLastError(), "timed step launch");
@@ -1696,8 +1826,8 @@ int lsf_graph_reset(lsf_engine* e) {
 // =============================================================================================
 // Batches: many independent engines stepped by shared launches. Each half-step is one launch of the bulk
 // kernel per kernel configuration over every member's tiles; the members' per-step operations are fused
-// by position (the q-th operation of a phase over all members is one slot: gathers and modal sources of a
-// slot become one launch each, sub-engines of a slot become a batch level of their own), and the DFT
+// by stage (stages_of; the q-th stage over all members is one slot: the gathers, the modal sources and the
+// jobs of a slot become one launch each, its sub-engines a batch level of their own), and the DFT
 // monitors of all members are sampled by one launch per source type.
 // =============================================================================================
 
@@ -1712,7 +1842,7 @@ struct KGroup {
 };
 
 struct Fused {
-  int kind = 0;  // OP_GATHER or OP_MODAL
+  int kind = 0;  // OP_GATHER, OP_MODAL, or any kind of k_jobs
   int cplx = 0;
   void* jobs = nullptr;
   lsf::Sched sc{};
@@ -1736,7 +1866,7 @@ struct DftLaunch {
 struct Level {
   std::vector<lsf_engine*> mem;
   std::vector<KGroup> hg, eg;
-  std::vector<Slot> slots[LSF_PH_BEFORE_H + 1];
+  std::vector<Slot> slots[3];  // as lsf_engine::stages
   std::vector<DftLaunch> dft;
   lsf::EnergyJob* energy = nullptr;
   int n_energy = 0;
@@ -1838,7 +1968,9 @@ int build_level(Level& L, const Tiling& t, int grid_blocks, bool sample, std::ve
                 std::vector<void*>& owned_groups);
 
 int build_slot(const std::vector<std::pair<lsf_engine*, Op>>& jobs, Slot& sl, std::vector<void*>& owned) {
-  // fusable kinds by field type; sub-engines as a level; the rest one by one
+  // fusable kinds by field type; jobs; sub-engines as a level; the rest one by one
+  std::vector<lsf::AnyJob> any;
+  std::vector<int> any_blocks;
   std::vector<std::pair<lsf_engine*, Op>> part[2][2];  // [gather, modal][float, c32]
   std::vector<lsf_engine*> subs;
   for (const auto& j : jobs) {
@@ -1847,10 +1979,20 @@ int build_slot(const std::vector<std::pair<lsf_engine*, Op>>& jobs, Slot& sl, st
       part[o.kind == OP_MODAL][j.first->cplx ? 1 : 0].push_back(j);
     else if (o.kind == OP_SUB_H || o.kind == OP_SUB_E)
       subs.push_back(o.sub);
-    else if (!((o.kind == OP_GATHER || o.kind == OP_MODAL) && o.n <= 0))
+    else if (is_job(o) && o.n > 0) {
+      any.push_back(any_job(j.first, o));
+      any_blocks.push_back((int)nblk(o.n, 256));
+    } else if (o.n > 0 || !(o.kind == OP_GATHER || o.kind == OP_MODAL || is_job(o)))
       sl.single.push_back(j);
   }
   int rc = LSF_OK;
+  if (!any.empty()) {
+    Fused f;
+    f.kind = OP_TAPE;
+    rc = dev_upload(any.data(), sizeof(any[0]) * any.size(), &f.jobs, owned);
+    if (!rc) rc = make_sched(any_blocks, &f.sc, owned);
+    if (!rc) sl.fused.push_back(f);
+  }
   for (int k = 0; k < 2 && !rc; ++k) {
     const int kind = k ? OP_MODAL : OP_GATHER;
     if (!part[k][0].empty()) rc = fuse_ops<float>(part[k][0], kind, sl, owned);
@@ -1902,20 +2044,20 @@ int build_sampling(Level& L, std::vector<void*>& owned) {
 int build_level(Level& L, const Tiling& t, int grid_blocks, bool sample, std::vector<void*>& owned,
                 std::vector<void*>& owned_groups) {
   int rc = build_groups(L, t, grid_blocks, owned_groups);
-  for (int ph = LSF_PH_CORRECT_H; ph <= LSF_PH_BEFORE_H && !rc; ++ph) {
-    std::vector<std::vector<std::pair<lsf_engine*, Op>>> by_pos;
+  for (int half = 0; half < 3 && !rc; ++half) {
+    std::vector<std::vector<std::pair<lsf_engine*, Op>>> stages;
     for (lsf_engine* e : L.mem) {
-      size_t q = 0;
-      for (const Op& o : e->ops) {
-        if (o.phase != ph || o.kind == OP_VIEW) continue;  // views run when the batch samples
-        if (o.sub ? joins(e, o.sub, t) : (o.in_bulk && flat_kernel(e, o.field, t))) continue;
-        if (by_pos.size() <= q) by_pos.resize(q + 1);
-        by_pos[q++].push_back({e, o});
+      auto taken = [&](const Op& o) { return o.sub ? joins(e, o.sub, t) : (o.in_bulk && flat_kernel(e, o.field, t)); };
+      std::vector<std::pair<int, const Op*>> at;
+      if ((rc = stages_of(e, half, taken, at))) return rc;
+      for (const auto& p : at) {
+        if ((int)stages.size() <= p.first) stages.resize(p.first + 1);
+        stages[p.first].push_back({e, *p.second});
       }
     }
-    for (const auto& jobs : by_pos) {
-      L.slots[ph].emplace_back();
-      if ((rc = build_slot(jobs, L.slots[ph].back(), owned))) break;
+    for (const auto& jobs : stages) {
+      L.slots[half].emplace_back();
+      if ((rc = build_slot(jobs, L.slots[half].back(), owned))) break;
     }
   }
   if (!rc && sample) rc = build_sampling(L, owned);
@@ -1931,6 +2073,8 @@ void run_slot(Slot& sl, bool h_half, hipStream_t s) {
     if (f.kind == OP_GATHER) {
       if (f.cplx) hipLaunchKernelGGL(lsf::k_gather_multi<c32>, grid, block, 0, s, (const lsf::GatherJob<c32>*)f.jobs, f.sc);
       else hipLaunchKernelGGL(lsf::k_gather_multi<float>, grid, block, 0, s, (const lsf::GatherJob<float>*)f.jobs, f.sc);
+    } else if (f.kind == OP_TAPE) {
+      hipLaunchKernelGGL(lsf::k_jobs, grid, block, 0, s, (const lsf::AnyJob*)f.jobs, f.sc);
     } else {
       if (f.cplx) hipLaunchKernelGGL(lsf::k_modal_multi<c32>, grid, block, 0, s, (const lsf::ModalJob<c32>*)f.jobs, f.sc);
       else hipLaunchKernelGGL(lsf::k_modal_multi<float>, grid, block, 0, s, (const lsf::ModalJob<float>*)f.jobs, f.sc);
@@ -1963,17 +2107,15 @@ void level_e_kernels(Level& L, hipStream_t s) {
 }
 
 void level_h_ops(Level& L, hipStream_t s) {
-  for (int ph = LSF_PH_CORRECT_H; ph <= LSF_PH_ADVANCE_H; ++ph)
-    for (Slot& sl : L.slots[ph]) run_slot(sl, true, s);
+  for (Slot& sl : L.slots[1]) run_slot(sl, true, s);
 }
 
 void level_e_ops(Level& L, hipStream_t s) {
-  for (int ph = LSF_PH_OFFDIAG; ph <= LSF_PH_ADVANCE_E; ++ph)
-    for (Slot& sl : L.slots[ph]) run_slot(sl, false, s);
+  for (Slot& sl : L.slots[2]) run_slot(sl, false, s);
 }
 
 void level_h(Level& L, hipStream_t s) {
-  for (Slot& sl : L.slots[LSF_PH_BEFORE_H]) run_slot(sl, true, s);
+  for (Slot& sl : L.slots[0]) run_slot(sl, true, s);
   level_h_kernels(L, s);
   level_h_ops(L, s);
 }
@@ -2111,7 +2253,7 @@ int lsf_batch_step_timed(lsf_batch* b, int n, void* stream, double* ms) {
     if ((rc = hip_check(hipEventCreate(&x), "event create"))) break;
   if (!rc) {
     for (int q = 0; q < n; ++q) {
-      for (Slot& sl : b->root.slots[LSF_PH_BEFORE_H]) run_slot(sl, true, s);
+      for (Slot& sl : b->root.slots[0]) run_slot(sl, true, s);
       (void)hipEventRecord(ev[4 * q + 0], s);
       level_h_kernels(b->root, s);
       (void)hipEventRecord(ev[4 * q + 1], s);

@@ -143,22 +143,31 @@ __global__ void k_table_view(int n, float* out, const float* __restrict__ tab, i
   out[r] = quintic(tab, counter[slot], i0[r], u0[r], base[r], m, cmax);
 }
 
-// Auxiliary 1D grid of a TFSF plane wave (tfsf.py:200-211). One block strides over the line.
-__global__ void k_line_h(int M, const float* __restrict__ E1, float* H1, const float* __restrict__ da,
-                         const float* __restrict__ db) {
-  for (int m = threadIdx.x; m < M - 1; m += blockDim.x) H1[m] = da[m] * H1[m] - db[m] * (E1[m + 1] - E1[m]);
+// Auxiliary 1D grid of a TFSF plane wave (tfsf.py:200-211), one thread per node.
+struct LineJob {
+  int M;
+  float* E1;
+  float* H1;
+  const float *ca, *cb, *da, *db;
+  int m_src;
+  const float* wave;
+  long long wave_len;
+  const long long* counter;
+  int slot;
+};
+
+__device__ __forceinline__ void line_h_row(const LineJob& J, long long m) {
+  if (m < J.M - 1) J.H1[m] = J.da[m] * J.H1[m] - J.db[m] * (J.E1[m + 1] - J.E1[m]);
 }
 
-__global__ void k_line_e(int M, float* E1, const float* __restrict__ H1, const float* __restrict__ ca,
-                         const float* __restrict__ cb, int m_src, const float* __restrict__ wave, long long wave_len,
-                         const long long* counter, int slot) {
-  const long long t = counter[slot];
-  const float w = (t >= 0 && t < wave_len) ? wave[t] : 0.f;
-  for (int m = 1 + threadIdx.x; m < M - 1; m += blockDim.x) {
-    float e = ca[m] * E1[m] - cb[m] * (H1[m] - H1[m - 1]);
-    if (m == m_src) e += w;
-    E1[m] = e;
+__device__ __forceinline__ void line_e_row(const LineJob& J, long long m) {
+  if (m < 1 || m >= J.M - 1) return;
+  float e = J.ca[m] * J.E1[m] - J.cb[m] * (J.H1[m] - J.H1[m - 1]);
+  if (m == J.m_src) {
+    const long long t = J.counter[J.slot];
+    e += (t >= 0 && t < J.wave_len) ? J.wave[t] : 0.f;
   }
+  J.E1[m] = e;
 }
 
 // Mixed (interface) ADE group, engine.py:743-791. State per node: D, E_prev, E_a, E_h[S], then per slot s and
@@ -562,8 +571,7 @@ struct TapeJob {
   const long long* counter;
 };
 
-__global__ void k_tape(TapeJob J) {
-  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void tape_row(const TapeJob& J, long long q) {
   if (q >= J.n) return;
   const long long slot = J.counter[0] - J.base[0];
   if (slot < 0 || slot >= J.n_slots) return;
@@ -594,8 +602,7 @@ struct GradJob {
   double* g;
 };
 
-__global__ void k_adj_grad(GradJob J) {
-  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void grad_row(const GradJob& J, long long q) {
   if (q >= J.n) return;
   const long long n = J.n_steps - 1 - J.counter[0];
   const long long slot = n - J.base[0];
@@ -623,8 +630,7 @@ struct AdjAdeJob {
   float* E;
 };
 
-__global__ void k_adj_ade_pre(AdjAdeJob J) {
-  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void ade_pre_row(const AdjAdeJob& J, long long q) {
   if (q >= J.n) return;
   const float* m = J.media + (long long)J.medium[q] * J.stride;
   const float inv = m[0];
@@ -645,8 +651,7 @@ __global__ void k_adj_ade_pre(AdjAdeJob J) {
   J.E[nd] = x;
 }
 
-__global__ void k_adj_ade_post(AdjAdeJob J) {
-  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void ade_post_row(const AdjAdeJob& J, long long q) {
   if (q >= J.n) return;
   J.E[J.node[q]] = J.save[q];
 }
@@ -676,8 +681,7 @@ struct AdjSrcJob {
   int stride;
 };
 
-__global__ void k_adj_src(AdjSrcJob J) {
-  const long long r = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void adj_src_row(const AdjSrcJob& J, long long r) {
   if (r >= J.n_rows) return;
   const long long n = J.h_side ? J.n_steps - J.counter[0] : J.n_steps - 1 - J.counter[1];
   if (n <= 0 || n % J.stride != 0) return;
@@ -694,6 +698,43 @@ __global__ void k_adj_src(AdjSrcJob J) {
     acc += v * (double)J.scale[q];
   }
   J.F[J.target[r]] += (float)acc;
+}
+
+// One launch over the rows of jobs of any of these kinds, of one engine or of many (blocks of 256 rows; sc maps each block
+// to its job). Each such launch costs 4.5-6 us whatever its size, and a batch of four designs made 24 a step of its
+// members' jobs one by one; the host puts jobs that do not touch each other's data into one launch.
+enum JobKind { JOB_TAPE, JOB_GRAD, JOB_ADE_PRE, JOB_ADE_POST, JOB_ADJ_SRC, JOB_LINE_H, JOB_LINE_E };
+
+struct AnyJob {
+  int kind;
+  long long rows;
+  union {
+    TapeJob tape;
+    GradJob grad;
+    AdjAdeJob ade;
+    AdjSrcJob src;
+    LineJob line;
+  };
+};
+
+__device__ __forceinline__ void job_row(const AnyJob& J, long long q) {
+  switch (J.kind) {
+    case JOB_TAPE: return tape_row(J.tape, q);
+    case JOB_GRAD: return grad_row(J.grad, q);
+    case JOB_ADE_PRE: return ade_pre_row(J.ade, q);
+    case JOB_ADE_POST: return ade_post_row(J.ade, q);
+    case JOB_ADJ_SRC: return adj_src_row(J.src, q);
+    case JOB_LINE_H: return line_h_row(J.line, q);
+    default: return line_e_row(J.line, q);
+  }
+}
+
+__global__ void k_job(AnyJob J) { job_row(J, (long long)blockIdx.x * blockDim.x + threadIdx.x); }
+
+__global__ void k_jobs(const AnyJob* __restrict__ jobs, Sched sc) {
+  int m, lt;
+  member_of(sc, blockIdx.x, m, lt);
+  job_row(jobs[m], (long long)lt * blockDim.x + threadIdx.x);
 }
 
 }  // namespace lsf
