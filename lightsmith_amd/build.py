@@ -5,6 +5,7 @@ Translation units (compiled by hipcc for gfx950 in parallel, then linked into li
   csrc/lsf_k_adj.hip the adjoint bulk kernels
   csrc/lsf_k_pass.hip the single-pass step kernel
   csrc/lsf_k_flat.hip the bulk H and E kernels of periodic engines
+  csrc/lsf_k_lean.hip the bulk H and E kernels of real engines without periodic axes, forward and adjoint
   csrc/lsf_k_h.hip the bulk H kernel instantiations, once per field type (float, complex64)
   csrc/lsf_k_e.hip the bulk E kernel instantiations, once per field type, material mode (dense, indexed)
                    and periodicity
@@ -31,7 +32,7 @@ ARCH = "gfx950"
 
 # (object name, source, extra defines)
 UNITS = [("lsf", "lsf.hip", []), ("k_adj", "lsf_k_adj.hip", []), ("k_pass", "lsf_k_pass.hip", []),
-         ("k_flat", "lsf_k_flat.hip", [])] + [
+         ("k_flat", "lsf_k_flat.hip", []), ("k_lean", "lsf_k_lean.hip", [])] + [
     (f"k_h_{t}", "lsf_k_h.hip", [f"-DLSF_H_CPLX={1 if t == 'c' else 0}", f"-DLSF_H_ENTRY=launch_update_h_{t}"])
     for t in ("f", "c")
 ] + [

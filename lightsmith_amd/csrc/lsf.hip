@@ -14,6 +14,7 @@
 
 #include "lsf.h"
 #include "lsf_launch.h"
+#include "lsf_lean.h"
 #include "lsf_pass.h"
 #include "lsf_sparse.h"
 
@@ -199,18 +200,60 @@ bool any_periodic(const lsf_engine* e) { return e->g.per[0] || e->g.per[1] || e-
 
 bool takes_flat(const Tiling& t) { return t.ry == 1 && t.waves == lsf::FLAT_WAVES; }
 
-// Engines with a periodic axis take the flat kernels for the one-row, four-wavefront tile shapes (what the drivers
-// and the default pick), except for the E update of D-form nodes.
+// Bytes a step of an engine goes over: fields, material, psi, pole state.
+long long step_bytes(const lsf_engine* e) {
+  const long long N = e->g.N, s = e->cplx ? 8 : 4;
+  long long psi = 0;
+  for (int f = 0; f < 2; ++f)
+    for (int ax = 0; ax < 3; ++ax)
+      if (e->pml[f][ax].prof) psi += 2 * s * (N / e->g.n[ax]) * e->pml[f][ax].ns;
+  return (6 * s + (e->mid ? 4 : 12)) * N + psi + 2 * s * e->n_ade * (long long)pole_regs(e);
+}
+constexpr long long MALL_BYTES = 256ll << 20;  // the memory-side cache
+
+// For the one-row, four-wavefront tile shapes (what the drivers and the default pick): engines with a periodic axis take
+// the flat kernels, except for the E update of D-form nodes; real engines without one take the lean kernels, except for
+// that update and for rows of a multiple of 64 cells past the memory-side cache, where the row kernels have neither
+// idle lanes nor instructions to save. Measured with 8 CPML cells and no poles, us per step (H + E), row -> lean kernels:
+// 60^3 16 -> 14, 131 x 117 x 150 56 -> 44, 200 x 160 x 140 80 -> 75, 239 x 201 x 181 181 -> 170, 336 x 300 x 270 533 -> 513; 256
+// x 256 x 128 161 -> 174, 256^3 307 -> 320, 320^3 582 -> 628. The adjoint's gain everywhere: 256 x 192 x 96 106 -> 93 (a
+// pass of the case 168.4 -> 159 ms), 4 designs of 14 million cells together 292 -> 237.
 bool flat_kernel(const lsf_engine* e, int field, const Tiling& t) {
-  return any_periodic(e) && !e->adjoint && takes_flat(t) && (field == 1 || pole_regs(e) == 0);
+  if (!takes_flat(t)) return false;
+  if (any_periodic(e)) return !e->adjoint && (field == 1 || pole_regs(e) == 0);
+  if (e->cplx || e->g.N >= (1ll << 30)) return false;
+  if (e->adjoint) return true;
+  return (field == 1 || pole_regs(e) == 0) && (e->g.n[0] % 64 != 0 || step_bytes(e) <= MALL_BYTES);
 }
 
 int flat_lpr(const lsf_engine* e) { return (e->g.n[0] + lsf::FLAT_CELLS - 1) / lsf::FLAT_CELLS; }
+
+int lean_tiles(const lsf_engine* e) {  // per plane
+  const int per = lsf::LEAN_OWN * lsf::LEAN_WAVES;
+  return (int)(((long long)e->g.n[0] * e->g.n[1] + per - 1) / per);
+}
+
+// Planes per tile of a lean launch over these engines. A plane carried in registers saves loads, short marches keep more
+// tiles' rows in the caches. Measured at 1 / 2 / 4 / 8 planes, us per step (H + E): 514 x 96 x 80 80 / 77 / 78 / 83, 200 x
+// 160 x 140 81 / 75 / 76 / 83, 256^3 354 / 323 / 320 / 334; 4 designs of 14 million cells, ms per run 251 / 232 / 229 / 234.
+int lean_planes(const lsf_engine* const* mem, int n) {
+  long long cells = 0;
+  for (int q = 0; q < n; ++q) cells += mem[q]->g.N;
+  int z = cells > (8ll << 20) ? 4 : 2;
+  auto blocks = [&]() {
+    long long b = 0;
+    for (int q = 0; q < n; ++q) b += (long long)lean_tiles(mem[q]) * ((mem[q]->g.n[2] + z - 1) / z);
+    return b;
+  };
+  while (z > 1 && blocks() < 1024) z /= 2;
+  return z;
+}
 
 // Planes per tile of a flat launch over these engines: 4 once that still leaves 16 wavefronts per SIMD (a plane
 // carried in registers saves two of ten loads), else 1. Measured at 1 / 2 / 4 planes: one 76 x 61 x 256 complex cell
 // 55 / 67 / 75 us per step, 12 cells of 50-98 x 50-98 x 256 521 / 516 / 515 us.
 int flat_planes(const lsf_engine* const* mem, int n) {
+  if (!any_periodic(mem[0])) return lean_planes(mem, n);
   long long waves = 0;
   for (int q = 0; q < n; ++q)
     waves += ((long long)flat_lpr(mem[q]) * mem[q]->g.n[1] + 63) / 64 * mem[q]->g.n[2];
@@ -242,6 +285,8 @@ StepArgs make_args(const lsf_engine* e, int field, const Tiling& t, int flat) {
   a.counter = e->counter;
   a.tick = e->tick;
   if (flat && !e->corr_off) a.corr = e->corr[field];
+  a.zlo = e->pass_z[0];
+  a.zhi = e->pass_z[1];
   const int rows = t.ry * t.waves * (64 / t.xw);
   a.tiles_x = (e->g.n[0] + t.xw - 1) / t.xw;
   a.tiles_y = (e->g.n[1] + rows - 1) / rows;
@@ -251,7 +296,7 @@ StepArgs make_args(const lsf_engine* e, int field, const Tiling& t, int flat) {
   if (flat) {
     a.zc = flat;
     a.lpr = flat_lpr(e);
-    a.tiles_x = (int)(((long long)a.lpr * e->g.n[1] + 64 * t.waves - 1) / (64 * t.waves));
+    a.tiles_x = any_periodic(e) ? (int)(((long long)a.lpr * e->g.n[1] + 64 * t.waves - 1) / (64 * t.waves)) : lean_tiles(e);
     a.tiles_y = 1;
   }
   const int tiles_z = (e->g.n[2] + a.zc - 1) / a.zc;
@@ -307,21 +352,18 @@ bool pass_eligible(const lsf_engine* e) {
 
 // Whether it is also the faster step. The pass moves fewer bytes but over two sets of E, H and H-side psi, so it gains
 // while both sets stay in the 256 MB memory-side cache, loses where only one does, and gains again where neither does
-// and it has pole state or rows off the 64-byte lines (its wavefronts cross row ends, the row kernels' do not). Measured
-// on boxes with 8 CPML cells, us per step, two kernels -> pass: 128 x 110 x 100, 3 poles 43 -> 32; 131 x 117 x 150 56 ->
-// 40; 192 x 160 x 128, 1 pole 73 -> 70 (both sets 240 MB); 200 x 160 x 140 81 -> 90 (182 and 300 MB); 514 x 96 x 80 77 ->
-// 89 (178 and 282 MB); 239 x 201 x 181, 2 poles 223 -> 177; 255 x 257 x 250, none 334 -> 308; 256^3, none 310 -> 309, 2
-// poles 389 -> 357; 320^3, none 576 -> 597, 3 poles 691 -> 667.
+// and it has pole state or rows off the 64-byte lines. Measured on boxes with 8 CPML cells, us per step, the two kernels
+// that the engine would take -> pass: 60^3 11.4 -> 8.9, 97^3 22 -> 18; 128 x 110 x 100, 3 poles 43 -> 32; 131 x 117 x 150
+// 40 -> 34; 192 x 160 x 128 66 -> 63 (both sets 260 MB), 1 pole 73 -> 64; 200 x 160 x 140 71 -> 85 (182 and 300 MB); 514 x
+// 96 x 80 73 -> 89 (178 and 282 MB); 239 x 201 x 181 168 -> 156, 2 poles 223 -> 177; 255 x 257 x 250 313 -> 308, 2 poles
+// 397 -> 351; 256^3 310 -> 309, 2 poles 389 -> 357; 320^3 576 -> 597, 3 poles 691 -> 664.
 bool pass_pays(const lsf_engine* e) {
-  const long long N = e->g.N, cache = 256ll << 20;
-  long long psi[2] = {0, 0};
-  for (int f = 0; f < 2; ++f)
-    for (int ax = 0; ax < 3; ++ax)
-      if (e->pml[f][ax].prof) psi[f] += 8 * (N / e->g.n[ax]) * e->pml[f][ax].ns;
-  const long long one = (24 + (e->mid ? 4 : 12)) * N + psi[0] + psi[1] + 8 * e->n_ade * (long long)pole_regs(e);
-  const long long both = one + 24 * N + psi[1];
-  if (both <= cache) return true;
-  return one > cache && (pole_regs(e) > 0 || e->g.n[0] % 16 != 0);
+  const long long N = e->g.N, one = step_bytes(e);
+  long long both = one + 24 * N;
+  for (int ax = 0; ax < 3; ++ax)
+    if (e->pml[1][ax].prof) both += 8 * (N / e->g.n[ax]) * e->pml[1][ax].ns;
+  if (both <= MALL_BYTES) return true;
+  return one > MALL_BYTES && (pole_regs(e) > 0 || e->g.n[0] % 16 != 0);
 }
 
 // Planes per tile of a pass. A tile begins with H of the plane below it, so more planes save work, while fewer make
@@ -375,18 +417,9 @@ lsf::PassArgs pass_args(const lsf_engine* e, int set) {
   return a;
 }
 
-// Arguments of the single pass, and the D-form chunk table.
-int sync_pass(lsf_engine* e, const StepArgs& ea) {
+// The planes between the z slabs.
+int plan_z(lsf_engine* e) {
   int rc = LSF_OK;
-  if (pole_regs(e) > 0) {
-    const long long n = 3ll * ea.nchunk * e->g.n[1] * e->g.n[2];
-    if (!e->dform) rc = hip_check(hipMalloc(&e->dform, sizeof(lsf::DChunk) * n), "hipMalloc D-form chunk table");
-    if (!rc) rc = hip_check(hipDeviceSynchronize(), "synchronize before the D-form chunk table");
-    if (rc) return rc;
-    lsf::launch_dform_chunks(ea, e->dform, n, nullptr);
-    if ((rc = hip_check(hipStreamSynchronize(nullptr), "D-form chunk table"))) return rc;
-  }
-  // the planes between the z slabs
   e->pass_z[0] = 0;
   e->pass_z[1] = e->g.n[2];
   for (int f = 0; f < 2; ++f) {
@@ -403,6 +436,20 @@ int sync_pass(lsf_engine* e, const StepArgs& ea) {
       if ((int)pr[k].w >= 0) hi = k;
     e->pass_z[0] = std::max(e->pass_z[0], lo);
     e->pass_z[1] = std::min(e->pass_z[1], hi);
+  }
+  return rc;
+}
+
+// Arguments of the single pass, and the D-form chunk table.
+int sync_pass(lsf_engine* e, const StepArgs& ea) {
+  int rc = LSF_OK;
+  if (pole_regs(e) > 0) {
+    const long long n = 3ll * ea.nchunk * e->g.n[1] * e->g.n[2];
+    if (!e->dform) rc = hip_check(hipMalloc(&e->dform, sizeof(lsf::DChunk) * n), "hipMalloc D-form chunk table");
+    if (!rc) rc = hip_check(hipDeviceSynchronize(), "synchronize before the D-form chunk table");
+    if (rc) return rc;
+    lsf::launch_dform_chunks(ea, e->dform, n, nullptr);
+    if ((rc = hip_check(hipStreamSynchronize(nullptr), "D-form chunk table"))) return rc;
   }
   if (!e->dev_pass) rc = hip_check(hipMalloc(&e->dev_pass, 2 * sizeof(lsf::PassArgs)), "hipMalloc pass arguments");
   if (rc) return rc;
@@ -506,6 +553,7 @@ int plan_corr(lsf_engine* e) {
     for (int* p : e->corr_rows) (void)hipFree(p);
     e->corr_rows.clear();
   }
+  if ((rc = plan_z(e))) return rc;
   if (!e->step_word && (rc = hip_check(hipMalloc(&e->step_word, sizeof(long long)), "hipMalloc step word"))) return rc;
   const int* n = e->g.n;
   const bool pass = pass_eligible(e);
@@ -515,7 +563,7 @@ int plan_corr(lsf_engine* e) {
     cs = lsf::Corrs{};
     cs.step = e->step_word;
     cs.z[0] = n[2];
-    if (!pass && !any_periodic(e)) continue;  // the row and the adjoint kernels make none
+    if (!pass && !flat_kernel(e, f, Tiling{1, lsf::FLAT_WAVES, 64, 1})) continue;  // the row kernels make none
     for (Op* po : in_order(e, f)) {
       Op& o = *po;
       if ((o.kind != OP_GATHER && o.kind != OP_MODAL) || o.field != f || o.phase == LSF_PH_OFFDIAG || cs.n == lsf::MAX_CORR ||
@@ -728,7 +776,7 @@ int sync_args(lsf_engine* e) {
   for (Op& o : e->ops) {
     if (o.kind != OP_SUB_H && o.kind != OP_SUB_E) continue;
     const lsf_engine* q = o.sub;
-    o.in_bulk = q->cplx == e->cplx && !q->mid == !e->mid && joins(e, o.sub, t) && joins(e, o.sub, own_tiling(q));
+    o.in_bulk = q->cplx == e->cplx && any_periodic(q) == any_periodic(e) && !q->mid == !e->mid && joins(e, o.sub, t) && joins(e, o.sub, own_tiling(q));
     if (o.in_bulk && o.kind == OP_SUB_H) mem.push_back(o.sub);
   }
   for (int f = 0; f < 2 && mem.size() > 1; ++f) {
@@ -1025,6 +1073,7 @@ int configurable(lsf_engine* e) {
   if (e->held) return fail(LSF_ESTATE, "the engine is held by a batch; destroy the batch before changing it");
   e->dirty = true;
   e->corr_planned = false;
+  e->pass_z[0] = e->pass_z[1] = 0;
   return LSF_OK;
 }
 
@@ -1836,7 +1885,7 @@ struct lsf_batch;
 namespace {
 
 struct KGroup {
-  int cplx = 0, per = 0, mat = 0, np = 0, adj = 0;
+  int cplx = 0, per = 0, mat = 0, np = 0, adj = 0, flat = 0;
   std::vector<lsf_engine*> mem;
   lsf::KLaunch L{};
 };
@@ -1904,9 +1953,11 @@ int build_groups(Level& L, const Tiling& t, int grid_blocks, std::vector<void*>&
       key.mat = field ? 0 : (e->mid ? 1 : 0);
       key.np = field ? 0 : pole_regs(e);
       key.adj = e->adjoint ? 1 : 0;
+      key.flat = flat_kernel(e, field, t);
       KGroup* g = nullptr;
       for (KGroup& x : groups)
-        if (x.cplx == key.cplx && x.per == key.per && x.mat == key.mat && x.np == key.np && x.adj == key.adj) g = &x;
+        if (x.cplx == key.cplx && x.per == key.per && x.mat == key.mat && x.np == key.np && x.adj == key.adj && x.flat == key.flat)
+          g = &x;
       if (!g) {
         groups.push_back(key);
         g = &groups.back();
@@ -1919,7 +1970,7 @@ int build_groups(Level& L, const Tiling& t, int grid_blocks, std::vector<void*>&
       if (g.adj) tg.xw = 64;
       std::vector<StepArgs> args;
       std::vector<int> counts;
-      const int flat = flat_kernel(g.mem[0], field, tg) ? flat_planes(g.mem.data(), (int)g.mem.size()) : 0;
+      const int flat = g.flat ? flat_planes(g.mem.data(), (int)g.mem.size()) : 0;
       for (lsf_engine* e : g.mem) {
         args.push_back(make_args(e, field, tg, flat));
         counts.push_back(args.back().nb);

@@ -31,6 +31,7 @@ void e_by_shape(const KLaunch& L, hipStream_t s) {
 }  // namespace
 
 void launch_adjoint_h(const KLaunch& L, hipStream_t s) {
+  if (L.flat) return launch_lean_h(L, true, s);
   if (L.ry == 2) {
     if (L.waves == 8) go_h<2, 8>(L, s);
     else go_h<2, 4>(L, s);
@@ -41,6 +42,7 @@ void launch_adjoint_h(const KLaunch& L, hipStream_t s) {
 }
 
 void launch_adjoint_e(const KLaunch& L, hipStream_t s) {
+  if (L.flat) return launch_lean_e(L, true, s);
   if (L.mat) e_by_shape<1>(L, s);
   else e_by_shape<0>(L, s);
 }

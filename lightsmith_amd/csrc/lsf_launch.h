@@ -18,7 +18,7 @@ struct KLaunch {
   int per;               // some axis periodic
   int mat;               // E: 1 = packed material ids, 0 = dense coefficients
   int np;                // E: pole registers (0 or the engine's max_poles, 1 to 4)
-  int flat = 0;          // the flat kernels (lsf_flat.h) instead of the row kernels
+  int flat = 0;          // the flat (periodic, lsf_flat.h) or lean (lsf_lean.h) kernels instead of the row kernels
 };
 
 // The tile shapes (rows per lane, wavefronts per block, x cells per row) with compiled kernels.
@@ -46,6 +46,10 @@ constexpr int FLAT_CELLS = 2, FLAT_WAVES = 4;
 void launch_flat_h(const KLaunch& L, hipStream_t s);
 void launch_flat_e(const KLaunch& L, hipStream_t s);
 
+// the lean kernels of real engines without periodic axes (lsf_lean.h)
+void launch_lean_h(const KLaunch& L, bool adjoint, hipStream_t s);
+void launch_lean_e(const KLaunch& L, bool adjoint, hipStream_t s);
+
 // the single-pass step (lsf_pass.h)
 struct PassArgs;
 struct PassLaunch {
@@ -62,13 +66,13 @@ void launch_adjoint_h(const KLaunch& L, hipStream_t s);
 void launch_adjoint_e(const KLaunch& L, hipStream_t s);
 
 inline void launch_update_h(const KLaunch& L, hipStream_t s) {
-  if (L.flat) return launch_flat_h(L, s);
+  if (L.flat) return L.per ? launch_flat_h(L, s) : launch_lean_h(L, false, s);
   if (L.cplx) launch_update_h_c(L, s);
   else launch_update_h_f(L, s);
 }
 
 inline void launch_update_e(const KLaunch& L, hipStream_t s) {
-  if (L.flat) return launch_flat_e(L, s);
+  if (L.flat) return L.per ? launch_flat_e(L, s) : launch_lean_e(L, false, s);
 #define LSF_PICK_E(T, M, P) \
   if ((L.cplx != 0) == (#T[0] == 'c') && L.mat == M && (L.per != 0) == (P != 0)) return launch_update_e_##T##M##P(L, s);
   LSF_E_LAUNCHERS(LSF_PICK_E)

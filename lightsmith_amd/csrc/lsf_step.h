@@ -70,6 +70,7 @@ struct StepArgs {
   int tiles_x, tiles_y, zc, nb, nbp;
   int lpr;               // lanes per x row of the flat kernels (tiles_x: their tiles per plane)
   Corrs corr;            // source corrections of this kernel's field
+  int zlo, zhi;          // planes [zlo, zhi) lie in no z slab of either field (lean kernels)
 };
 
 // The tiles of one launch: every member's tiles laid end to end.
