@@ -140,7 +140,7 @@ class Batch:
             return self.chunk, False
         stream = torch.cuda.Stream(device=self._dev)
         stream.wait_stream(torch.cuda.current_stream(self._dev))
-        state = {"captured": False}
+        state = {"captured": False, "last": None}
         self._graph_stream = stream
 
         def run():
@@ -152,10 +152,11 @@ class Batch:
                 state["captured"] = True
                 self._graphed = True
                 return
-            stream.wait_stream(torch.cuda.current_stream(self._dev))
-            check(self.lib.lsf_batch_graph_replay(self._h, 1, ctypes.c_void_p(stream.cuda_stream)),
-                  "lsf_batch_graph_replay")
-            torch.cuda.current_stream(self._dev).wait_stream(stream)
+            cur = torch.cuda.current_stream(self._dev)  # on the caller's stream, as Engine.make_runner
+            if state["last"] is not None and state["last"] != cur:
+                cur.wait_stream(state["last"])
+            state["last"] = cur
+            check(self.lib.lsf_batch_graph_replay(self._h, 1, ctypes.c_void_p(cur.cuda_stream)), "lsf_batch_graph_replay")
             self._advance(self.stride)
 
         return run, True

@@ -888,7 +888,7 @@ class Engine:
             return self.chunk, False
         stream = torch.cuda.Stream(device=self._dev)
         stream.wait_stream(torch.cuda.current_stream(self._dev))
-        state = {"captured": False}
+        state = {"captured": False, "last": None}
         self._graph_stream = stream
 
         def run():
@@ -900,9 +900,13 @@ class Engine:
                 state["captured"] = True
                 self._graphed = True
                 return
-            stream.wait_stream(torch.cuda.current_stream(self._dev))
-            check(self.lib.lsf_graph_replay(self._h, 1, ctypes.c_void_p(stream.cuda_stream)), "lsf_graph_replay")
-            torch.cuda.current_stream(self._dev).wait_stream(stream)
+            # replayed on the caller's stream: a side stream costs two event waits a chunk. A stream other than the last
+            # one waits for it, as the replays of one graph follow one another.
+            cur = torch.cuda.current_stream(self._dev)
+            if state["last"] is not None and state["last"] != cur:
+                cur.wait_stream(state["last"])
+            state["last"] = cur
+            check(self.lib.lsf_graph_replay(self._h, 1, ctypes.c_void_p(cur.cuda_stream)), "lsf_graph_replay")
             self.n_host += self.stride
 
         return run, True
