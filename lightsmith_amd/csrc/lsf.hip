@@ -211,6 +211,16 @@ long long step_bytes(const lsf_engine* e) {
 }
 constexpr long long MALL_BYTES = 256ll << 20;  // the memory-side cache
 
+// Tiles an XCD takes in a row (Sched::win) in the launches of steps over so many bytes. Up to the memory-side cache each
+// XCD keeps to a range of its own, whose data its L2 may still hold from the last launch; past it the XCDs advance
+// through the grid together, so that DRAM serves eight neighbouring runs instead of eight distant ones. Measured, ranges
+// of their own -> windows of 8 / 16 / 32, us per step: 320^3, 3 poles (pass) 664 -> 627 / 628 / 626, 255 x 257 x 250, 2
+// poles (pass) 350 -> 327 / 323 / 333, 192 x 160 x 128, 1 pole (pass, 240 MB) 69 -> 63 / - / 63, 256^3 (H + E) 305 -> 294 / - /
+// 299; but 200 x 160 x 140 (182 MB) 74 -> 76 / 76 / -, 120 x 110 x 100 25 -> 26 / 26 / -, 97^3 34 -> 35 / 35 / -. Per run, 12
+// complex and real cells 15.8 -> 15.4 / 15.3 / 15.2 ms, 4 designs 231 -> 223 / 224 / 225 ms, the adjoint of a 256 x 192 x
+// 96 waveguide (217 MB) 159 -> 153 / 155 / - ms.
+int window(long long bytes) { return bytes > (200ll << 20) ? 16 : 0; }
+
 // For the one-row, four-wavefront tile shapes (what the drivers and the default pick): engines with a periodic axis take
 // the flat kernels, except for the E update of D-form nodes; real engines without one take the lean kernels, except for
 // that update and for rows of a multiple of 64 cells past the memory-side cache, where the row kernels have neither
@@ -350,30 +360,32 @@ bool pass_eligible(const lsf_engine* e) {
   return e->g.N < (1ll << 30);
 }
 
-// Whether it is also the faster step. The pass moves fewer bytes but over two sets of E, H and H-side psi, so it gains
-// while both sets stay in the 256 MB memory-side cache, loses where only one does, and gains again where neither does
-// and it has pole state or rows off the 64-byte lines. Measured on boxes with 8 CPML cells, us per step, the two kernels
-// that the engine would take -> pass: 60^3 11.4 -> 8.9, 97^3 22 -> 18; 128 x 110 x 100, 3 poles 43 -> 32; 131 x 117 x 150
-// 40 -> 34; 192 x 160 x 128 66 -> 63 (both sets 260 MB), 1 pole 73 -> 64; 200 x 160 x 140 71 -> 85 (182 and 300 MB); 514 x
-// 96 x 80 73 -> 89 (178 and 282 MB); 239 x 201 x 181 168 -> 156, 2 poles 223 -> 177; 255 x 257 x 250 313 -> 308, 2 poles
-// 397 -> 351; 256^3 310 -> 309, 2 poles 389 -> 357; 320^3 576 -> 597, 3 poles 691 -> 664.
-bool pass_pays(const lsf_engine* e) {
-  const long long N = e->g.N, one = step_bytes(e);
-  long long both = one + 24 * N;
+long long second_bytes(const lsf_engine* e) {  // the second set of a pass
+  long long b = 24 * e->g.N;
   for (int ax = 0; ax < 3; ++ax)
-    if (e->pml[1][ax].prof) both += 8 * (N / e->g.n[ax]) * e->pml[1][ax].ns;
-  if (both <= MALL_BYTES) return true;
-  return one > MALL_BYTES && (pole_regs(e) > 0 || e->g.n[0] % 16 != 0);
+    if (e->pml[1][ax].prof) b += 8 * (e->g.N / e->g.n[ax]) * e->pml[1][ax].ns;
+  return b;
+}
+
+// Whether it is also the faster step. The pass moves fewer bytes but over two sets of E, H and H-side psi: it gains while
+// both sets stay in the 256 MB memory-side cache and where not even one does, and loses between. Measured on boxes with
+// 8 CPML cells, us per step, the two kernels that the engine would take -> pass: 60^3 11.4 -> 8.9, 97^3 22 -> 18; 131 x 117
+// x 150 40 -> 34; 192 x 160 x 128 66 -> 63 (both sets 260 MB), 1 pole 73 -> 60; 200 x 160 x 140 70 -> 78 (182 and 300 MB);
+// 514 x 96 x 80 72 -> 78 (178 and 282 MB); 256^3 299 -> 275, 255 x 257 x 250 291 -> 272, 2 poles 397 -> 314; 336 x 300 x 270
+// 474 -> 444; 320^3 550 -> 540, 3 poles 648 -> 613.
+bool pass_pays(const lsf_engine* e) {
+  const long long one = step_bytes(e);
+  return one + second_bytes(e) <= MALL_BYTES || one > MALL_BYTES;
 }
 
 // Planes per tile of a pass. A tile begins with H of the plane below it, so more planes save work, while fewer make
 // tiles whose cells the caches still hold for their neighbours, and D-form rounds hide more of the first. Measured, us per
-// step at 2 / 4 / 8 / 16 planes: no poles, 120 x 110 x 100 27 / 29 / 27 / 32, 200 x 160 x 140 85 / 90 / 93 / 106, 256^3
-// 312 / 309 / 330 / 348; 2 poles per D-form node, 240 x 200 x 180 189 / 175 / 183 / 204, 256^3 399 / 358 / 357 / 379; 1
-// pole, 400 x 300 x 260 664 / 578 / 558 / 592. Small grids take fewer, down to one, while the blocks number less than
-// four per compute unit (40 x 36 x 32, 3 poles: 13.2 at 1, 15.4 at 2, the step's dipole and sampling included).
+// step at 2 / 4 / 8: no poles, 120 x 110 x 100 27 / 29 / 27, 131 x 117 x 150 42 / 43 / -, 200 x 160 x 140 78 / 79 / 91, 256^3
+// 284 / 275 / 298, 320^3 550 / 540 / 555; 2 poles per D-form node, 240 x 200 x 180 175 / 155 / 161, 255 x 257 x 250 353 / 314
+// / 320; 3 poles, 320^3 720 / 614 / 613. Small grids take fewer, down to one, while the blocks number less than four per
+// compute unit (40 x 36 x 32, 3 poles: 13.2 at 1, 15.4 at 2, with the step's dipole and sampling).
 int pass_planes(const lsf_engine* e, int tiles_p) {
-  int z = pole_regs(e) == 0 ? 2 : e->g.N >= (12ll << 20) ? 8 : 4;
+  int z = pole_regs(e) == 0 ? (step_bytes(e) <= MALL_BYTES ? 2 : 4) : e->g.N >= (24ll << 20) ? 8 : 4;
   while (z > 1 && (long long)tiles_p * ((e->g.n[2] + z - 1) / z) < 1024) z /= 2;
   return z;
 }
@@ -804,6 +816,7 @@ void launch_pass_step(lsf_engine* e, int set, hipStream_t s) {
   lsf::PassLaunch L{};
   L.args = e->dev_pass + set;
   L.sc = lsf::Sched{nullptr, nullptr, e->pass_nb, (e->pass_nb + 7) / 8 * 8, set ? e->rev_e : 0};
+  L.sc.win = window(step_bytes(e) + second_bytes(e));
   L.mat = e->mid ? 1 : 0;
   L.np = pole_regs(e);
   for (int f = 0; f < 2; ++f)
@@ -818,6 +831,7 @@ lsf::KLaunch own_launch(lsf_engine* e, int field) {
   L.args = (e->args_override ? e->args_override : e->dev_args) + field;
   L.sc = lsf::Sched{nullptr, nullptr, e->nb[field], e->nbp[field]};
   L.grid = e->nbp[field];
+  L.sc.win = window(step_bytes(e));
   L.ry = e->ry;
   L.waves = e->waves;
   L.xw = e->xw;
@@ -1944,6 +1958,8 @@ int build_groups(Level& L, const Tiling& t, int grid_blocks, std::vector<void*>&
   for (lsf_engine* e : L.mem)
     for (const Op& o : e->ops)
       if (o.kind == OP_SUB_H && joins(e, o.sub, t)) mem.push_back(o.sub);
+  long long bytes = 0;
+  for (const lsf_engine* e : mem) bytes += step_bytes(e);
   for (int field = 0; field < 2; ++field) {
     std::vector<KGroup>& groups = field ? L.hg : L.eg;
     for (lsf_engine* e : mem) {
@@ -1980,6 +1996,7 @@ int build_groups(Level& L, const Tiling& t, int grid_blocks, std::vector<void*>&
       if (rc) return rc;
       g.L.args = (const StepArgs*)da;
       if ((rc = make_sched(counts, &g.L.sc, owned))) return rc;
+      g.L.sc.win = window(bytes);
       g.L.grid = g.L.sc.n_pad;
       if (grid_blocks > 0 && !g.adj) g.L.grid = std::min(g.L.sc.n_pad, (grid_blocks + 7) / 8 * 8);
       g.L.ry = tg.ry;

@@ -200,7 +200,7 @@ __device__ __forceinline__ void ah_tile(const StepArgs& a, int t) {
 
 template <int RY, int WAVES>
 __global__ void __launch_bounds__(64 * WAVES) k_adjoint_h(const StepArgs* __restrict__ args, Sched sc) {
-  const int t = xcd_tile(blockIdx.x, sc.n_pad);
+  const int t = tile_of(blockIdx.x, sc);
   if (t >= sc.n_tiles) return;
   int m, lt;
   member_of(sc, t, m, lt);
@@ -418,7 +418,7 @@ __device__ __forceinline__ void ae_tile(const StepArgs& a, int t, const float* t
 template <int MAT, int RY, int WAVES>
 __global__ void __launch_bounds__(64 * WAVES) k_adjoint_e(const StepArgs* __restrict__ args, Sched sc) {
   __shared__ float tab[MAT == 1 ? 256 : 1];
-  const int t = xcd_tile(blockIdx.x, sc.n_pad, sc.rev);
+  const int t = tile_of(blockIdx.x, sc);
   if (t >= sc.n_tiles) return;
   int m, lt;
   member_of(sc, t, m, lt);

@@ -658,7 +658,7 @@ __device__ __forceinline__ void e_tile(const StepArgs& a, int t, const float* ta
 template <class T, int V, int WAVES, bool LOOP>
 __global__ void __launch_bounds__(64 * WAVES) k_flat_h(const StepArgs* __restrict__ args, Sched sc) {
   for (int b = blockIdx.x; b < sc.n_pad; b += gridDim.x) {
-    const int t = xcd_tile(b, sc.n_pad, sc.rev);
+    const int t = tile_of(b, sc);
     if (t < sc.n_tiles) {
       int m, lt;
       member_of(sc, t, m, lt);
@@ -675,7 +675,7 @@ __global__ void __launch_bounds__(64 * WAVES) k_flat_e(const StepArgs* __restric
   __shared__ float tab[MAT == 1 ? 256 : 1];
   int cur = -1;
   for (int b = blockIdx.x; b < sc.n_pad; b += gridDim.x) {
-    const int t = xcd_tile(b, sc.n_pad, sc.rev);
+    const int t = tile_of(b, sc);
     if (t >= sc.n_tiles) {
       if (!LOOP) break;
       continue;

@@ -586,7 +586,7 @@ __device__ __forceinline__ void ae_tile(const StepArgs& a, int t, const float* t
 template <bool ADJ, bool LOOP>
 __global__ void __launch_bounds__(64 * LEAN_WAVES) k_lean_h(const StepArgs* __restrict__ args, Sched sc) {
   for (int b = blockIdx.x; b < sc.n_pad; b += gridDim.x) {
-    const int t = xcd_tile(b, sc.n_pad, sc.rev);
+    const int t = tile_of(b, sc);
     if (t < sc.n_tiles) {
       int m, lt;
       member_of(sc, t, m, lt);
@@ -606,7 +606,7 @@ __global__ void __launch_bounds__(64 * LEAN_WAVES) k_lean_e(const StepArgs* __re
   __shared__ float tab[MAT == 1 ? 256 : 1];
   int cur = -1;
   for (int b = blockIdx.x; b < sc.n_pad; b += gridDim.x) {
-    const int t = xcd_tile(b, sc.n_pad, sc.rev);
+    const int t = tile_of(b, sc);
     if (t >= sc.n_tiles) {
       if (!LOOP) break;
       continue;

@@ -561,7 +561,7 @@ __global__ void __launch_bounds__(64 * PASS_WAVES) k_pass(const PassArgs* __rest
   __shared__ float tab[MAT == 1 ? 256 : 1];
   __shared__ float4 med_tab[NP > 0 ? MAX_MEDIA_VEC4 : 1];
   __shared__ pass::Nodes nodes[NP > 0 ? PASS_WAVES : 1];
-  const int t = xcd_tile(blockIdx.x, sc.n_pad, sc.rev);
+  const int t = tile_of(blockIdx.x, sc);
   if (t >= sc.n_tiles) return;  // whole block
   int m, lt;
   member_of(sc, t, m, lt);

@@ -80,7 +80,16 @@ struct Sched {
   int n_tiles;
   int n_pad;           // n_tiles rounded up to a multiple of 8 (the period of the XCD-aware order)
   int rev = 0;         // each XCD walks its tile range backwards (xcd_tile)
+  int win = 0;         // tiles an XCD takes in a row before the launch moves on to the next 8 win tiles; 0: one range each
 };
+
+// The tile of block b (xcd_tile), by windows where the launch asks for them.
+__device__ __forceinline__ int tile_of(int b, const Sched& sc) {
+  if (sc.win == 0) return xcd_tile(b, sc.n_pad, sc.rev);
+  const int per = 8 * sc.win, q = sc.rev ? sc.n_pad - 1 - b : b;
+  const int w = q / per, r = q - w * per, left = min(per, sc.n_pad - w * per);
+  return w * per + (r & 7) * (left >> 3) + (r >> 3);
+}
 
 // D-form media table in device memory: n_media * (2 + 3 * max_poles) floats
 // ({1/eps_inf, poles, c1 c2 c3 of each pole}, zeros past a medium's poles)
@@ -356,7 +365,7 @@ __device__ __forceinline__ void h_tile(const StepArgs& a, int t) {
 template <class T, int RY, int WAVES, int XW, bool PER, bool LOOP>
 __global__ void __launch_bounds__(64 * WAVES) k_update_h(const StepArgs* __restrict__ args, Sched sc) {
   for (int b = blockIdx.x; b < sc.n_pad; b += gridDim.x) {
-    const int t = xcd_tile(b, sc.n_pad, sc.rev);
+    const int t = tile_of(b, sc);
     if (t < sc.n_tiles) {
       int m, lt;
       member_of(sc, t, m, lt);
@@ -766,7 +775,7 @@ __global__ void __launch_bounds__(64 * WAVES) k_update_e(const StepArgs* __restr
   __shared__ float4 med_tab[NP > 0 ? MAX_MEDIA_VEC4 : 1];
   int cur = -1;
   for (int b = blockIdx.x; b < sc.n_pad; b += gridDim.x) {
-    const int t = xcd_tile(b, sc.n_pad, sc.rev);
+    const int t = tile_of(b, sc);
     if (t >= sc.n_tiles) {
       if (!LOOP) break;
       continue;
