@@ -108,7 +108,7 @@ class AdjointProblem:
         if any(getattr(g, "w", None) is not None or hasattr(g, "slot_vert") for g in groups):
             raise ValueError("the adjoint transposes pure D-form groups only (no mixed or vertex-tensor groups)")
         self.fwd = Engine(device, shape=shape, dx=dx, dt=dt, single=True, inv_eps=inv_eps, groups=groups, pml=pml,
-                          sources=sources, monitors=[monitor], dft_stride=self.stride, material="dense", fused=False)
+                          sources=sources, monitors=[monitor], dft_stride=self.stride, material="dense")
         ry, waves, _, zc = filling_tiling([self.fwd.shape])
         tiling = (ry, waves, 64, zc)  # the adjoint kernels take 64-cell rows
         self.fwd.set_tiling(*tiling)
