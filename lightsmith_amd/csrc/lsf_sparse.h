@@ -444,6 +444,21 @@ struct DftJob {
   float* partial;  // per-block energy partials of this monitor, or null
 };
 
+// acc[q][p] += ph[q] v over the frequencies, eight at a time: a group's accumulators are loaded before any is stored.
+// Bound by the accumulators' traffic; one by one every load waited for the store before it (a chunk's sampling of a 320^3
+// scene's plane 32 -> 27 us, its energy sum 28 -> 20 us; a gold sphere's 81 wavelengths, per pass 5028 -> 4933 us).
+__device__ __forceinline__ void dft_add(c32* __restrict__ acc, const c32* ph, int nf, long long np, long long p, c32 v) {
+  constexpr int G = 8;
+  for (int q0 = 0; q0 < nf; q0 += G) {
+    c32 a[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) a[g] = acc[min(q0 + g, nf - 1) * np + p];
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+      if (q0 + g < nf) acc[(q0 + g) * np + p] = add(a[g], mul(ph[q0 + g], v));
+  }
+}
+
 template <class S>
 __device__ __forceinline__ void dft_block(const DftJob<S>& J, int blk, c32* ph, float* red) {
   const double te = (double)J.counter[0] * J.dt;
@@ -461,19 +476,11 @@ __device__ __forceinline__ void dft_block(const DftJob<S>& J, int blk, c32* ph, 
   if (p < np) {
     const S se = J.esrc[J.eidx[p]];
     e2 += norm2(se);
-    for (int q = 0; q < nf; ++q) {
-      const c32 v = mul(ph[q], to_c(se));
-      c32 a = J.acc_e[q * np + p];
-      J.acc_e[q * np + p] = add(a, v);
-    }
+    dft_add(J.acc_e, ph, nf, np, p, to_c(se));
     if (J.acc_h) {
       const S sh = scl(0.5f, add(J.hsrc[J.h1[p]], J.hsrc[J.h2[p]]));
       e2 += norm2(sh);
-      for (int q = 0; q < nf; ++q) {
-        const c32 v = mul(ph[nf + q], to_c(sh));
-        c32 a = J.acc_h[q * np + p];
-        J.acc_h[q * np + p] = add(a, v);
-      }
+      dft_add(J.acc_h, ph + nf, nf, np, p, to_c(sh));
     }
   }
   if (J.partial) {  // the block's sum of |E|^2 (+ |H|^2): a butterfly within each wavefront, then the wavefronts'
@@ -524,8 +531,17 @@ __device__ __forceinline__ void energy_sum(const EnergyJob& J) {
   for (int m = 0; m < J.n_mon; ++m) {
     const int g = J.mon_group[m];
     if (g < 0) continue;
+    // one thread keeps the order of the sum; sixteen partials are loaded at a time
     double s = 0.0;
-    for (int q = J.mon_off[m]; q < J.mon_off[m + 1]; ++q) s += J.partial[q];
+    const int q1 = J.mon_off[m + 1];
+    for (int q = J.mon_off[m]; q < q1; q += 16) {
+      float v[16];
+#pragma unroll
+      for (int t = 0; t < 16; ++t) v[t] = J.partial[min(q + t, q1 - 1)];
+#pragma unroll
+      for (int t = 0; t < 16; ++t)
+        if (q + t < q1) s += v[t];
+    }
     tot[g] += s;
     have[g] = 1;
   }
