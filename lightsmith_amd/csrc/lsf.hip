@@ -689,19 +689,21 @@ int apart(const Op& a, const Op& b, bool* yes) {
   } else if ((h_src(a) && e_side(b)) || (h_src(b) && e_side(a))) {
     *yes = true;
   } else if (e_side(a) && e_side(b) && a.kind != b.kind) {
-    std::vector<long long> t[2] = {std::vector<long long>(a.n), std::vector<long long>(b.n)};
-    for (int q = 0; q < 2; ++q) {
-      const Op& o = q ? b : a;
-      if (int rc = hip_check(hipMemcpy(t[q].data(), o.target, sizeof(long long) * o.n, hipMemcpyDeviceToHost), "operation nodes"))
-        return rc;
-      std::sort(t[q].begin(), t[q].end());
-    }
-    size_t i = 0, j = 0;
+    const Op& few = a.n <= b.n ? a : b;  // a bit for every index in the smaller set's range
+    const Op& many = a.n <= b.n ? b : a;
+    std::vector<long long> t(few.n), u(many.n);
+    int rc = LSF_OK;
+    if (few.n > 0) rc = hip_check(hipMemcpy(t.data(), few.target, sizeof(long long) * few.n, hipMemcpyDeviceToHost), "operation nodes");
+    if (!rc && few.n > 0)
+      rc = hip_check(hipMemcpy(u.data(), many.target, sizeof(long long) * many.n, hipMemcpyDeviceToHost), "operation nodes");
+    if (rc) return rc;
     *yes = true;
-    while (i < t[0].size() && j < t[1].size() && *yes) {
-      *yes = t[0][i] != t[1][j];
-      if (t[0][i] < t[1][j]) ++i;
-      else ++j;
+    if (few.n > 0) {
+      const auto ends = std::minmax_element(t.begin(), t.end());
+      const long long lo = *ends.first, hi = *ends.second;
+      std::vector<bool> has(hi - lo + 1, false);
+      for (long long v : t) has[v - lo] = true;
+      for (long long v : u) *yes = *yes && !(v >= lo && v <= hi && has[v - lo]);
     }
   }
   return LSF_OK;

@@ -400,24 +400,34 @@ class Engine:
             self.fused_table_tensor = not hit.size and self.lib.lsf_fuse_table_tensor(self._h) == 0
         self._graph_stream = None
         self._graphed = False
-        # single-pass stepping: a second set of E, H and H-side psi that the step alternates with; the state is in the
-        # first whenever the host has control, so the second is scratch (24 bytes a cell)
-        self._two_sets = False
-        can = 0 if _sub else self.lib.lsf_can_pair(self._h)  # 1: it could, 2: and it is the faster step
-        if (can == 2 and Engine.single_pass) if fused is None else (can and fused):
-            try:
-                sets = [torch.empty_like(self.E_flat), torch.empty_like(self.H_flat)] + \
-                    [torch.empty(n, dtype=self.fdt, device=self._dev) if n else None for n in self._psiH_size]
-            except torch.cuda.OutOfMemoryError:  # the two-kernel step needs no second set
-                if fused:
-                    raise
-                sets = None
-            if sets is not None:
-                self._keep += [t for t in sets if t is not None]
-                arr = (ctypes.c_void_p * 3)(*[None if t is None else t.data_ptr() for t in sets[2:]])
-                give = self.lib.lsf_set_fused if fused else self.lib.lsf_set_pair
-                check(give(self._h, ptr(sets[0]), ptr(sets[1]), arr), "lsf_set_pair")
-                self._two_sets = True
+        # single-pass stepping (_second_set): taken at once if asked for, else when the engine first steps by itself
+        self._two_sets, self._pair_open = False, not _sub and fused is not False
+        self._fused = bool(fused)
+        if fused:
+            self._second_set()
+
+    def _second_set(self):
+        """Give the engine a second set of E, H and H-side psi if single passes over two sets are its faster step (or
+        asked for). The state is in the first set whenever the host has control, so the second is scratch, 24 bytes a
+        cell; members of a batch never need it."""
+        if not self._pair_open or self._held or self._graphed:
+            return
+        self._pair_open = False
+        can = self.lib.lsf_can_pair(self._h)  # 1: it could, 2: and it is the faster step
+        if not (can if self._fused else can == 2 and Engine.single_pass):
+            return
+        try:
+            sets = [torch.empty_like(self.E_flat), torch.empty_like(self.H_flat)] + \
+                [torch.empty(n, dtype=self.fdt, device=self._dev) if n else None for n in self._psiH_size]
+        except torch.cuda.OutOfMemoryError:  # the two-kernel step needs no second set
+            if self._fused:
+                raise
+            return
+        self._keep += [t for t in sets if t is not None]
+        arr = (ctypes.c_void_p * 3)(*[None if t is None else t.data_ptr() for t in sets[2:]])
+        give = self.lib.lsf_set_fused if self._fused else self.lib.lsf_set_pair
+        check(give(self._h, ptr(sets[0]), ptr(sets[1]), arr), "lsf_set_pair")
+        self._two_sets = True
 
     def set_tiling(self, rows_per_lane: int, waves: int, x_cells: int, z_chunk: int):
         """Launch tiling of this engine's bulk kernels (lsf_set_tiling); before a graph is captured."""
@@ -867,10 +877,12 @@ class Engine:
 
     # --- stepping (engine.py:665-719) ------------------------------------------------------------
     def step(self):
+        self._second_set()
         check(self.lib.lsf_step(self._h, 1, self._stream()), "lsf_step")
         self.n_host += 1
 
     def steps(self, n: int):
+        self._second_set()
         check(self.lib.lsf_step(self._h, int(n), self._stream()), "lsf_step")
         self.n_host += int(n)
 
@@ -878,12 +890,14 @@ class Engine:
         check(self.lib.lsf_sample(self._h, self._stream()), "lsf_sample")
 
     def chunk(self):
+        self._second_set()
         check(self.lib.lsf_chunk(self._h, 1, self.stride, self._stream()), "lsf_chunk")
         self.n_host += self.stride
 
     def make_runner(self, use_graphs: bool):
         """(run_one_chunk, used_graphs): with graphs, one chunk is captured as a HIP graph on a side stream
         and replayed (engine.py:685-709; the warm-up chunk runs eagerly)."""
+        self._second_set()
         if not use_graphs:
             return self.chunk, False
         stream = torch.cuda.Stream(device=self._dev)

@@ -66,9 +66,12 @@ def test_the_pass_is_taken_by_working_set(gpu):
     work between the H and the E update never do."""
     ns = cases.product_ns()
     small = cases.dispersive_box(ns, gpu, shape=(30, 28, 26))
+    assert not small._two_sets  # not before it steps by itself
+    small.step()
     assert small._two_sets
-    assert not cases.dispersive_box(ns, gpu, shape=(30, 28, 26), fused=False)._two_sets
-    assert not cases.tfsf_box(ns, gpu)._two_sets
+    for e in (cases.dispersive_box(ns, gpu, shape=(30, 28, 26), fused=False), cases.tfsf_box(ns, gpu)):
+        e.step()
+        assert not e._two_sets
     old = ns.Engine.tiling
     ns.Engine.tiling = (2, 4, 64, 8)
     try:
