@@ -97,7 +97,9 @@ int lsf_set_ade(lsf_engine* eng, const int32_t* dev_chunk_base, void* dev_P, int
  * Replaces the off-diagonal rows (engine.py:653-655), the 1D-fed TFSF corrections (tfsf.py:195-204)
  * and the Bloch plane corrections (tfsf.py:274-286). dev_scale (or NULL = 1) scales each row's sum: 1/eps_inf
  * for a pure D-form E node, where the reference's correction enters through D before the group update.
- * dev_src NULL reads the engine's own H (its current buffer, see lsf_set_fused). */
+ * dev_src NULL reads the engine's own H (its current buffer, see lsf_set_fused). Gathers and modal sources may be
+ * made by the bulk kernels: dev_target is then read when the engine first steps after a configuration call (the other
+ * arrays at every step). */
 int lsf_add_gather(lsf_engine* eng, int phase, int field, int64_t n_rows, int width, const int64_t* dev_target,
                    const void* dev_src, const int64_t* dev_src_idx, const void* dev_w, const float* dev_scale);
 

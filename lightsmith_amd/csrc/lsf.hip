@@ -227,7 +227,7 @@ int window(long long bytes) { return bytes > (200ll << 20) ? 16 : 0; }
 // idle lanes nor instructions to save. Measured with 8 CPML cells and no poles, us per step (H + E), row -> lean kernels:
 // 60^3 16 -> 14, 131 x 117 x 150 56 -> 44, 200 x 160 x 140 80 -> 75, 239 x 201 x 181 181 -> 170, 336 x 300 x 270 533 -> 513; 256
 // x 256 x 128 161 -> 174, 256^3 307 -> 320, 320^3 582 -> 628. The adjoint's gain everywhere: 256 x 192 x 96 106 -> 93 (a
-// pass of the case 168.4 -> 159 ms), 4 designs of 14 million cells together 292 -> 237.
+// gradient of 800 steps 168.4 -> 159 ms), 4 designs of 14 million cells together 292 -> 237.
 bool flat_kernel(const lsf_engine* e, int field, const Tiling& t) {
   if (!takes_flat(t)) return false;
   if (any_periodic(e)) return !e->adjoint && (field == 1 || pole_regs(e) == 0);

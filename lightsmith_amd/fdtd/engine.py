@@ -2,7 +2,7 @@
 
 The constructor takes the reference's arguments (shape, dx, dt, single, inv_eps, groups, pml, sources,
 monitors, dft_stride, periodic, bloch, offdiag, time_monitors, mirror, widths) and hands the time stepping
-to the HIP library ``_lsf.so``: one H kernel and one E kernel per step (curl + CPML fused, the pure-ADE
+to the HIP library ``_lsf.so``: one H kernel and one E kernel per step, or both in one (curl + CPML fused, the pure-ADE
 update fused into the E kernel), plus sparse kernels for sources, interface groups and monitors.
 Host set-up runs once in NumPy (float64) and uploads float32 tables.
 
