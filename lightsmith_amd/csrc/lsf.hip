@@ -575,7 +575,8 @@ int plan_corr(lsf_engine* e) {
     cs = lsf::Corrs{};
     cs.step = e->step_word;
     cs.z[0] = n[2];
-    if (!pass && !flat_kernel(e, f, Tiling{1, lsf::FLAT_WAVES, 64, 1})) continue;  // the row kernels make none
+    // the row kernels and the adjoint ones make none
+    if (e->adjoint || (!pass && !flat_kernel(e, f, Tiling{1, lsf::FLAT_WAVES, 64, 1}))) continue;
     for (Op* po : in_order(e, f)) {
       Op& o = *po;
       if ((o.kind != OP_GATHER && o.kind != OP_MODAL) || o.field != f || o.phase == LSF_PH_OFFDIAG || cs.n == lsf::MAX_CORR ||

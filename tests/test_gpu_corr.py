@@ -136,3 +136,27 @@ def test_corrections_in_a_batch(gpu):
         for x, y in zip(a.state_tensors(), b.state_tensors()):
             assert torch.equal(x, y)
     batch.close()
+
+
+@pytest.mark.parametrize("tiling", [(1, 4, 64, 4), (2, 4, 64, 4)])
+def test_corrections_of_an_adjoint_engine(gpu, tiling):
+    """An adjoint engine's gathers and modal sources run, whatever the tile shape: lsf_step, lsf_step_noalloc and a batch agree."""
+    from lightsmith_amd import _lib
+    from lightsmith_amd.fdtd.batch import Batch
+    from tests.test_zz_no_alloc import _bind
+    lib, ns = _lib.load(), cases.product_ns()
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    a, b, m, bare = (_engine(ns, gpu, (17, 12, 15), ops, tiling=tiling, fused=False) for ops in [LISTS[1]] * 3 + [[]])
+    for e in (a, b, m, bare):
+        _lib.check(lib.lsf_set_adjoint(e._h, 1), "lsf_set_adjoint")
+    batch = Batch([m], schedule=tiling + (0,))
+    for n in (1, 4):
+        a.steps(n)
+        bare.steps(n)
+        batch.steps(n)
+        _lib.check(_bind(lib)(b._h, n, stream), "lsf_step_noalloc")
+    torch.cuda.synchronize()
+    for x, y, z in zip(a.state_tensors(), b.state_tensors(), m.state_tensors()):
+        assert torch.equal(x, y) and torch.equal(x, z)
+    assert not torch.equal(a.E_flat, bare.E_flat) and not torch.equal(a.H_flat, bare.H_flat)
+    batch.close()
