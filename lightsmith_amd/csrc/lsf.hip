@@ -652,20 +652,31 @@ int plan_corr(lsf_engine* e) {
   return LSF_OK;
 }
 
+// Whether an operation gathers from a field of an engine.
+bool gathers_from(const Op& o, const lsf_engine* e, int field) {
+  const char* f = (const char*)(field ? e->H : e->E);
+  const char* src = (const char*)o.src;
+  return o.kind == OP_GATHER && src >= f && src < f + (size_t)(3 * e->g.N) * (e->cplx ? 8 : 4);
+}
+
 // Whether a sub-engine's bulk updates can run inside its engine's launches (under tiling t): flat kernels on both sides, no
-// launch of its own left, and nothing between the engine's update and its own but corrections that the engine's kernel
-// makes without reading what the sub-engine's writes. A Bloch plane source's 3 x 3 column, whose H and E launches took
+// launch of its own left, nothing between the engine's update and its own but corrections that the engine's kernel makes,
+// and no correction that reads what the same launch writes: one of the engine's or of a sub-engine joined before it the
+// sub-engine's field, one of the sub-engine's theirs. A Bloch plane source's 3 x 3 column, whose H and E launches took
 // 5 us a step each beside the engine's 17.
 bool joins(lsf_engine* e, lsf_engine* sub, const Tiling& t) {
+  auto reads = [](const lsf_engine* by, const lsf_engine* of, int f) {
+    for (const Op& o : by->ops)
+      if (o.field == f && gathers_from(o, of, f)) return true;
+    return false;
+  };
   for (int f = 0; f < 2; ++f) {
     if (!flat_kernel(e, f, t) || !flat_kernel(sub, f, t)) return false;
-    const char* w = (const char*)(f ? sub->H : sub->E);
-    const size_t size = (size_t)(3 * sub->g.N) * (sub->cplx ? 8 : 4);
+    if (reads(sub, e, f)) return false;
     for (const Op* o : in_order(e, f)) {
       if (o->sub == sub) break;
-      if (o->sub ? !joins(e, o->sub, t) : !o->in_bulk) return false;
-      const char* src = (const char*)o->src;
-      if (o->kind == OP_GATHER && src >= w && src < w + size) return false;
+      if (o->sub ? !joins(e, o->sub, t) || reads(sub, o->sub, f) || reads(o->sub, sub, f) : !o->in_bulk) return false;
+      if (gathers_from(*o, sub, f)) return false;
     }
   }
   for (const Op& o : sub->ops)
