@@ -662,9 +662,10 @@ bool gathers_from(const Op& o, const lsf_engine* e, int field) {
 // Whether a sub-engine's bulk updates can run inside its engine's launches (under tiling t): flat kernels on both sides, no
 // launch of its own left, nothing between the engine's update and its own but corrections that the engine's kernel makes,
 // and no correction that reads what the same launch writes: one of the engine's or of a sub-engine joined before it the
-// sub-engine's field, one of the sub-engine's theirs. A Bloch plane source's 3 x 3 column, whose H and E launches took
-// 5 us a step each beside the engine's 17.
+// sub-engine's field, one of the sub-engine's theirs. An adjoint engine's update is another kernel. A Bloch plane source's
+// 3 x 3 column, whose H and E launches took 5 us a step each beside the engine's 17.
 bool joins(lsf_engine* e, lsf_engine* sub, const Tiling& t) {
+  if (e->adjoint || sub->adjoint) return false;
   auto reads = [](const lsf_engine* by, const lsf_engine* of, int f) {
     for (const Op& o : by->ops)
       if (o.field == f && gathers_from(o, of, f)) return true;

@@ -61,3 +61,29 @@ def test_sub_engines_that_read_their_engine_or_each_other(gpu, links, bloch):
         assert torch.equal(x, y) and torch.equal(x, z), q
     assert a.E_flat.abs().max() > 0 and torch.isfinite(a.E_flat.abs()).all()
     batch.close()
+
+
+@pytest.mark.parametrize("which", [0, 1])
+def test_a_sub_engine_on_the_other_side_of_an_adjoint(gpu, which):
+    """A forward sub-engine of an adjoint engine (0) and an adjoint one of a forward engine (1) step their own update."""
+    from lightsmith_amd import _lib
+    ns, out = cases.product_ns(), []
+    for tiling in ((1, 4, 64, 4), (2, 4, 64, 4)):
+        old = ns.Engine.tiling
+        ns.Engine.tiling = tiling
+        try:
+            make = lambda s, **kw: cases.make(ns, gpu, shape=s, dx=2.0, dt=0.9 * 2.0 / np.sqrt(3), fused=False,  # noqa: E731
+                                              inv_eps=np.full((3,) + s, 1 / 2.25), pml=ns.PMLSpec(cells=((2, 2),) * 3), **kw)
+            eng = make((17, 12, 15))
+            sub = make((9, 8, 11), _sub=True, _counter=eng._counter)
+        finally:
+            ns.Engine.tiling = old
+        _lib.check(eng.lib.lsf_set_adjoint((eng, sub)[which]._h, 1), "lsf_set_adjoint")
+        eng.add_subengine(sub)
+        for e in (eng, sub):
+            cases.random_fields(e, 3)
+        eng.steps(5)
+        out.append(eng)
+    torch.cuda.synchronize()
+    for q, (x, y) in enumerate(zip(*(e.state_tensors() for e in out))):
+        assert torch.equal(x, y), q
