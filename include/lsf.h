@@ -211,7 +211,7 @@ int lsf_sample(lsf_engine* eng, void* stream);
 int lsf_chunk(lsf_engine* eng, int n_chunks, int stride, void* stream);
 
 /* HIP graph of one chunk (make_runner, engine.py:685-709): capture on `stream` (not the legacy default
- * stream), replay n times, drop. */
+ * stream), replay n times, drop. A replay after a step with a changed configuration captures again first. */
 int lsf_graph_capture(lsf_engine* eng, int stride, void* stream);
 int lsf_graph_replay(lsf_engine* eng, int n, void* stream);
 int lsf_graph_reset(lsf_engine* eng);

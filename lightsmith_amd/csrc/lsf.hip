@@ -145,6 +145,10 @@ struct lsf_engine {
   int rev_e = 1;  // the E launch walks each XCD's tiles backwards (lsf_set_tile_order)
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
+  int graph_stride = 0;
+  long long plan = 0;        // how often what launches name (arguments, plans, row tables) was made anew
+  long long sub_plan = 0;    // the sub-engines' (plan_of), as the arguments of joined launches hold it
+  long long graph_plan = 0;  // plan_of the engine, as the captured graph holds it
   lsf::StepArgs* dev_args = nullptr;  // library scratch: [0] E kernel, [1] H kernel arguments
   const lsf::StepArgs* args_override = nullptr;  // during lsf_step_noalloc: the arguments staged in `scratch`
   lsf::StepArgs host_args[2];          // lsf_step_noalloc: host source of the staged arguments (outlives the copy)
@@ -560,6 +564,7 @@ std::vector<Op*> in_order(lsf_engine* e, int field) {  // what runs after a fiel
 int plan_corr(lsf_engine* e) {
   if (e->corr_planned) return LSF_OK;
   int rc = LSF_OK;
+  ++e->plan;
   if (!e->corr_rows.empty()) {
     if ((rc = hip_check(hipDeviceSynchronize(), "synchronize before planning corrections"))) return rc;
     for (int* p : e->corr_rows) (void)hipFree(p);
@@ -773,16 +778,24 @@ int plan_stages(lsf_engine* e) {
   return LSF_OK;
 }
 
+// Changes whenever memory that launches of the engine or of its sub-engines name may have been freed or filled anew.
+long long plan_of(const lsf_engine* e) {
+  long long p = e->plan;
+  for (const Op& o : e->ops)
+    if (o.kind == OP_SUB_H) p += plan_of(o.sub);
+  return p;
+}
+
 // Upload the engine's kernel arguments (and its sub-engines') when its configuration changed. Not called
 // during graph capture.
 int sync_args(lsf_engine* e) {
   for (const Op& o : e->ops)
-    if (o.kind == OP_SUB_H) {
-      if (o.sub->dirty) e->dirty = true;
-      const int rc = sync_args(o.sub);
-      if (rc) return rc;
-    }
-  if (!e->dirty) return LSF_OK;
+    if (o.kind == OP_SUB_H)
+      if (const int rc = sync_args(o.sub)) return rc;
+  if (!e->dirty && plan_of(e) - e->plan == e->sub_plan) return LSF_OK;
+  e->dirty = true;  // until all of it is done
+  ++e->plan;
+  e->sub_plan = plan_of(e) - e->plan;
   int rc = LSF_OK;
   if (!e->dev_args) rc = hip_check(hipMalloc(&e->dev_args, 2 * sizeof(StepArgs)), "hipMalloc kernel arguments");
   else if (e->launched) rc = hip_check(hipDeviceSynchronize(), "synchronize before an argument update");
@@ -1809,7 +1822,7 @@ int lsf_chunk(lsf_engine* e, int n_chunks, int stride, void* stream) {
 }  // extern "C"
 
 namespace {
-int capture_chunk(lsf_engine* e, int stride, hipStream_t s, hipGraph_t* graph, hipGraphExec_t* exec) {
+int capture_chunk(lsf_engine* e, int stride, hipStream_t s) {
   int rc = hip_check(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "begin capture");
   if (rc) return rc;
   run_steps(e, stride, s);
@@ -1817,13 +1830,36 @@ int capture_chunk(lsf_engine* e, int stride, hipStream_t s, hipGraph_t* graph, h
   hipGraph_t g = nullptr;
   rc = hip_check(hipStreamEndCapture(s, &g), "end capture");
   if (rc) return rc;
-  *graph = g;
-  rc = hip_check(hipGraphInstantiate(exec, g, nullptr, nullptr, 0), "graph instantiate");
+  e->graph = g;
+  rc = hip_check(hipGraphInstantiate(&e->exec, g, nullptr, nullptr, 0), "graph instantiate");
   if (rc) {
     (void)hipGraphDestroy(g);
-    *graph = nullptr;
-    *exec = nullptr;
+    e->graph = nullptr;
+    e->exec = nullptr;
   }
+  e->graph_stride = stride;
+  e->graph_plan = plan_of(e);
+  return rc;
+}
+
+int drop_graph(lsf_engine* e) {
+  int rc = LSF_OK;
+  if (e->exec || e->graph) rc = hip_check(hipDeviceSynchronize(), "synchronize before graph reset");
+  if (e->exec) (void)hipGraphExecDestroy(e->exec);
+  if (e->graph) (void)hipGraphDestroy(e->graph);
+  e->exec = nullptr;
+  e->graph = nullptr;
+  return rc;
+}
+
+// The graph again, after a change of the configuration has freed what it names.
+int capture_again(lsf_engine* e) {
+  int rc = drop_graph(e);
+  if (!rc) rc = sync_args(e);
+  hipStream_t s = nullptr;
+  if (!rc) rc = hip_check(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), "capture stream");
+  if (!rc) rc = capture_chunk(e, e->graph_stride, s);
+  if (s) (void)hipStreamDestroy(s);
   return rc;
 }
 }  // namespace
@@ -1837,13 +1873,14 @@ int lsf_graph_capture(lsf_engine* e, int stride, void* stream) {
   if (!e->cbd && !e->mid) return fail(LSF_ESTATE, "no material set");
   if (stride < 1) return fail(LSF_EINVAL, "stride must be >= 1");
   if (int rc1 = sync_args(e)) return rc1;
-  hipStream_t s = (hipStream_t)stream;
-  return capture_chunk(e, stride, s, &e->graph, &e->exec);
+  return capture_chunk(e, stride, (hipStream_t)stream);
 }
 
 int lsf_graph_replay(lsf_engine* e, int n, void* stream) {
   if (valid(e)) return LSF_EINVAL;
   if (!e->exec) return fail(LSF_ESTATE, "no captured graph");
+  if (plan_of(e) != e->graph_plan)
+    if (int rc = capture_again(e)) return rc;
   for (int q = 0; q < n; ++q) {
     const int rc = hip_check(hipGraphLaunch(e->exec, (hipStream_t)stream), "graph launch");
     if (rc) return rc;
@@ -1890,13 +1927,7 @@ int lsf_set_fused(lsf_engine* e, void* E2, void* H2, void* const* psiH2) {
 
 int lsf_graph_reset(lsf_engine* e) {
   if (valid(e)) return LSF_EINVAL;
-  int rc = LSF_OK;
-  if (e->exec || e->graph) rc = hip_check(hipDeviceSynchronize(), "synchronize before graph reset");
-  if (e->exec) (void)hipGraphExecDestroy(e->exec);
-  if (e->graph) (void)hipGraphDestroy(e->graph);
-  e->exec = nullptr;
-  e->graph = nullptr;
-  return rc;
+  return drop_graph(e);
 }
 
 }  // extern "C"
