@@ -2082,9 +2082,9 @@ int build_level(Level& L, const Tiling& t, int grid_blocks, bool sample, std::ve
                 std::vector<void*>& owned_groups);
 
 int build_slot(const std::vector<std::pair<lsf_engine*, Op>>& jobs, Slot& sl, std::vector<void*>& owned) {
-  // fusable kinds by field type; jobs; sub-engines as a level; the rest one by one
-  std::vector<lsf::AnyJob> any;
-  std::vector<int> any_blocks;
+  // fusable kinds by field type; jobs; sub-engines as a level; the rest one by one. Members' gradients that are added to
+  // the same array take turns: one launch after another, in the members' order.
+  std::vector<std::vector<lsf::AnyJob>> turns;
   std::vector<std::pair<lsf_engine*, Op>> part[2][2];  // [gather, modal][float, c32]
   std::vector<lsf_engine*> subs;
   for (const auto& j : jobs) {
@@ -2094,18 +2094,26 @@ int build_slot(const std::vector<std::pair<lsf_engine*, Op>>& jobs, Slot& sl, st
     else if (o.kind == OP_SUB_H || o.kind == OP_SUB_E)
       subs.push_back(o.sub);
     else if (is_job(o) && o.n > 0) {
-      any.push_back(any_job(j.first, o));
-      any_blocks.push_back((int)nblk(o.n, 256));
+      const lsf::AnyJob J = any_job(j.first, o);
+      size_t at = 0;
+      for (size_t q = 0; q < turns.size() && J.kind == lsf::JOB_GRAD; ++q)
+        for (const lsf::AnyJob& x : turns[q])
+          if (x.kind == lsf::JOB_GRAD && x.grad.g < J.grad.g + J.rows && J.grad.g < x.grad.g + x.rows) at = q + 1;
+      if (turns.size() <= at) turns.resize(at + 1);
+      turns[at].push_back(J);
     } else if (o.n > 0 || !(o.kind == OP_GATHER || o.kind == OP_MODAL || is_job(o)))
       sl.single.push_back(j);
   }
   int rc = LSF_OK;
-  if (!any.empty()) {
+  for (const std::vector<lsf::AnyJob>& any : turns) {
+    std::vector<int> blocks;
+    for (const lsf::AnyJob& J : any) blocks.push_back((int)nblk(J.rows, 256));
     Fused f;
     f.kind = OP_TAPE;
     rc = dev_upload(any.data(), sizeof(any[0]) * any.size(), &f.jobs, owned);
-    if (!rc) rc = make_sched(any_blocks, &f.sc, owned);
-    if (!rc) sl.fused.push_back(f);
+    if (!rc) rc = make_sched(blocks, &f.sc, owned);
+    if (rc) return rc;
+    sl.fused.push_back(f);
   }
   for (int k = 0; k < 2 && !rc; ++k) {
     const int kind = k ? OP_MODAL : OP_GATHER;

@@ -105,3 +105,33 @@ def test_batch_operations_sharing_launches(gpu):
             assert torch.equal(x, y)
     batch.close()
     b2.close()
+
+
+def test_members_of_a_batch_that_share_a_gradient(gpu):
+    """Adjoint engines whose gradients are added to one array, as for an objective over several runs of a design: the members'
+    terms in their order, step by step, as one engine after another adds them."""
+    from lightsmith_amd import _lib
+    from lightsmith_amd.fdtd.batch import Batch
+    case = cases.adjoint_case(steps=40, stride=8)
+    make = lambda: [_adjoint(gpu, case, seed=s) for s in (5, 6, 7)]  # noqa: E731
+    alone, mem = make(), make()
+    shared = []
+    for probs in (alone, mem):
+        n = alone[0].n_nodes
+        both = torch.zeros(2 * n, dtype=torch.float64, device=gpu)  # the third's gradient overlaps half of the others'
+        for p, at in zip(probs, (0, 0, n // 2)):
+            _lib.check(p.fwd.lib.lsf_add_adjoint_gradient(p.adj._h, n, _lib.ptr(p._nodes), _lib.ptr(p.cb_design), _lib.ptr(p.tape),
+                                                          p.n_slots, _lib.ptr(p.base), p.n_steps, _lib.ptr(both[at:])),
+                       "lsf_add_adjoint_gradient")
+            p.adj.set_tiling(1, 4, 64, 8)
+        shared.append(both)
+    batch = Batch([p.adj for p in mem], schedule=(1, 4, 64, 8, 0))
+    for _ in range(33):
+        batch.steps(1)
+        for p in alone:
+            p.adj.steps(1)
+    torch.cuda.synchronize()
+    assert torch.equal(*shared) and shared[0].abs().max() > 0
+    for p, m in zip(alone, mem):
+        assert torch.equal(p.g, m.g)
+    batch.close()
