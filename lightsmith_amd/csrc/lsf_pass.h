@@ -18,7 +18,7 @@
 // one-pole nodes hold one (265 a cell, D-form rounds and slabs included). So:
 // - every address is a wave-uniform base and a 32-bit lane offset; the three row offsets advance by a plane per
 //   iteration (a component is below 4 GB), nothing else is recomputed;
-// - lanes outside a CPML slab take a profile that adds nothing, whole wavefronts outside one skip its terms;
+// - lanes outside a CPML slab read a psi that they do not use, whole wavefronts outside one skip its terms;
 // - D-form nodes are advanced by node, not by cell: the owners of a plane's nodes list them in LDS, the lanes take 64
 //   at a time.
 // Two cells per lane halve the instructions but take 150-200 registers (320^3, 3 poles: 742 us against 667), two rows
@@ -97,11 +97,6 @@ __device__ __forceinline__ float hide(float x) {
   return x;
 }
 
-// A profile whose psi stays zero and adds nothing, in place of "not in the slab" (index -1)
-__device__ __forceinline__ float4 slab_or_none(const float4 p) {
-  return (int)p.w >= 0 ? p : make_float4(0.f, 0.f, 1.f, -1.f);
-}
-
 __device__ __forceinline__ cbytes in_bytes(const void* p) { return (cbytes)as_global((const char*)p); }
 __device__ __forceinline__ bytes out_bytes(void* p) { return (bytes)as_global((char*)p); }
 
@@ -135,14 +130,14 @@ __device__ __forceinline__ void tile(const PassArgs& a, int t, const float* tab,
   // CPML of the lane: x, and y of its row and the row below
   const float4* q;
   q = a.prof[0][0];
-  const float4 pex = slab_or_none(q ? ((const float4*)as_global(q))[i] : no_pml());
+  const float4 pex = q ? ((const float4*)as_global(q))[i] : no_pml();
   q = a.prof[1][0];
-  const float4 phx = slab_or_none(q ? ((const float4*)as_global(q))[i] : no_pml());
+  const float4 phx = q ? ((const float4*)as_global(q))[i] : no_pml();
   q = a.prof[0][1];
-  const float4 pey = slab_or_none(q ? ((const float4*)as_global(q))[j] : no_pml());
+  const float4 pey = q ? ((const float4*)as_global(q))[j] : no_pml();
   q = a.prof[1][1];
-  const float4 phy = slab_or_none(q ? ((const float4*)as_global(q))[j] : no_pml());
-  const float4 phy0 = slab_or_none(q ? ((const float4*)as_global(q))[max(j - 1, 0)] : no_pml());
+  const float4 phy = q ? ((const float4*)as_global(q))[j] : no_pml();
+  const float4 phy0 = q ? ((const float4*)as_global(q))[max(j - 1, 0)] : no_pml();
   const bool has_xh = __ballot(phx.w >= 0.f) != 0ull, has_xe = __ballot(pex.w >= 0.f) != 0ull;
   const bool has_yh = __ballot(phy.w >= 0.f || phy0.w >= 0.f) != 0ull, has_ye = __ballot(pey.w >= 0.f) != 0ull;
 
@@ -157,6 +152,11 @@ __device__ __forceinline__ void tile(const PassArgs& a, int t, const float* tab,
   // coefficients would be kept in a register each.)
   auto pml = [](float acc, const float4 pr, float coef, float der, float& psi) {
     return acc + pml_apply(make_float4(pr.x, hide(pr.y), KAP ? hide(pr.z) : pr.z, pr.w), KAP, coef, der, psi);
+  };
+  // the same along x or y, for the lanes in the slab
+  auto pml_in = [&](float acc, const float4 pr, float coef, float der, float& psi) {
+    const float v = pml(acc, pr, coef, der, psi);
+    return pr.w >= 0.f ? v : acc;
   };
   // psi offsets: x slabs [k][j][p], y slabs [k][p][i], z slabs [p][j][i] (o: the cell's offset on plane k)
   auto xoff = [&](int f, const float4 pr, int k, int jj) {
@@ -236,14 +236,14 @@ __device__ __forceinline__ void tile(const PassArgs& a, int t, const float* tab,
     {
       const float da = azu - az, db = y1 - ay;
       float acc = -cH * (da - db);
-      if (has_yh) acc = pml(acc, phy, -cH, da, qy);
+      if (has_yh) acc = pml_in(acc, phy, -cH, da, qy);
       if (iz >= 0) acc = pml(acc, pz, cH, db, qz0);
       hxq = hx + acc;
     }
     {
       const float azr = shfl_dn(az), da = x1 - ax, db = azr - az;
       float acc = -cH * (da - db);
-      if (has_xh) acc = pml(acc, phx, cH, db, qx);
+      if (has_xh) acc = pml_in(acc, phx, cH, db, qx);
       if (iz >= 0) acc = pml(acc, pz, -cH, da, qz1);
       hyq = hy + acc;
     }
@@ -331,8 +331,8 @@ __device__ __forceinline__ void tile(const PassArgs& a, int t, const float* tab,
       float acc = -cH * (da - db), acc0 = -cH * (da0 - db0);
       if (has_yh) {
         float n = qxy, n0 = qxy0;
-        acc = pml(acc, phy, -cH, da, n);
-        acc0 = pml(acc0, phy0, -cH, da0, n0);
+        acc = pml_in(acc, phy, -cH, da, n);
+        acc0 = pml_in(acc0, phy0, -cH, da0, n0);
         qxy = st ? n : qxy;
       }
       if (izh >= 0) {
@@ -350,7 +350,7 @@ __device__ __forceinline__ void tile(const PassArgs& a, int t, const float* tab,
       float acc = -cH * (da - db);
       if (has_xh) {
         float n = qyx;
-        acc = pml(acc, phx, cH, db, n);
+        acc = pml_in(acc, phx, cH, db, n);
         qyx = st ? n : qyx;
       }
       if (izh >= 0) {
@@ -366,14 +366,14 @@ __device__ __forceinline__ void tile(const PassArgs& a, int t, const float* tab,
       float acc = -cH * (da - db), acc0 = -cH * (da0 - db0);
       if (has_xh) {
         float n = qzx, n0 = qzx0;
-        acc = pml(acc, phx, -cH, da, n);
-        acc0 = pml(acc0, phx, -cH, da0, n0);
+        acc = pml_in(acc, phx, -cH, da, n);
+        acc0 = pml_in(acc0, phx, -cH, da0, n0);
         qzx = st ? n : qzx;
       }
       if (has_yh) {
         float n = qzy, n0 = qzy0;
-        acc = pml(acc, phy, cH, db, n);
-        acc0 = pml(acc0, phy0, cH, db0, n0);
+        acc = pml_in(acc, phy, cH, db, n);
+        acc0 = pml_in(acc0, phy0, cH, db0, n0);
         qzy = st ? n : qzy;
       }
       hz1 = st ? hz1 + acc : hz1;
@@ -447,7 +447,7 @@ __device__ __forceinline__ void tile(const PassArgs& a, int t, const float* tab,
       float acc = c * (da - db);
       if (has_ye) {
         float n = sxy;
-        acc = pml(acc, pey, c, da, n);
+        acc = pml_in(acc, pey, c, da, n);
         sxy = st ? n : sxy;
       }
       if (ize >= 0) {
@@ -463,7 +463,7 @@ __device__ __forceinline__ void tile(const PassArgs& a, int t, const float* tab,
       float acc = c * (da - db);
       if (has_xe) {
         float n = syx;
-        acc = pml(acc, pex, -c, db, n);
+        acc = pml_in(acc, pex, -c, db, n);
         syx = st ? n : syx;
       }
       if (ize >= 0) {
@@ -479,12 +479,12 @@ __device__ __forceinline__ void tile(const PassArgs& a, int t, const float* tab,
       float acc = c * (da - db);
       if (has_xe) {
         float n = szx;
-        acc = pml(acc, pex, c, da, n);
+        acc = pml_in(acc, pex, c, da, n);
         szx = st ? n : szx;
       }
       if (has_ye) {
         float n = szy;
-        acc = pml(acc, pey, -c, db, n);
+        acc = pml_in(acc, pey, -c, db, n);
         szy = st ? n : szy;
       }
       ew = finish(2, st, w1, acc);
