@@ -408,6 +408,7 @@ lsf::PassArgs pass_args(const lsf_engine* e, int set) {
     for (int f = 0; f < 2; ++f) {
       a.prof[f][ax] = e->pml[f][ax].prof;
       a.ns[f][ax] = e->pml[f][ax].ns;
+      a.has_k[f][ax] = e->pml[f][ax].has_k;
     }
     for (int c = 0; c < 3; ++c) {
       a.psiE[ax][c] = (float*)e->pml[0][ax].psi[c];
@@ -847,8 +848,11 @@ void launch_pass_step(lsf_engine* e, int set, hipStream_t s) {
   L.sc.win = window(step_bytes(e) + second_bytes(e));
   L.mat = e->mid ? 1 : 0;
   L.np = pole_regs(e);
+  bool with = false, without = false;
   for (int f = 0; f < 2; ++f)
-    for (int ax = 0; ax < 3; ++ax) L.kappa |= e->pml[f][ax].prof && e->pml[f][ax].has_k;
+    for (int ax = 0; ax < 3; ++ax)
+      if (e->pml[f][ax].prof) (e->pml[f][ax].has_k ? with : without) = true;
+  L.kappa = with ? (without ? 2 : 1) : 0;
   lsf::launch_pass(L, s);
   e->launched = true;
   use_set(e, set ^ 1);

@@ -1,5 +1,5 @@
 // Instantiations of the single-pass step kernel (lsf_pass.h): material mode x poles per D-form node (the slot
-// stride) x CPML with kappa.
+// stride) x the kappa term (on no axis, on every axis with CPML, on some).
 
 #include "lsf_launch.h"
 #include "lsf_pass.h"
@@ -29,8 +29,10 @@ __global__ void k_dform_chunks(StepArgs a, DChunk* out, long long n) {
 
 template <int MAT, int NP>
 void go(const PassLaunch& L, hipStream_t s) {
-  if (L.kappa) hipLaunchKernelGGL((k_pass<MAT, NP, true>), dim3(L.sc.n_pad), dim3(64 * PASS_WAVES), 0, s, L.args, L.sc);
-  else hipLaunchKernelGGL((k_pass<MAT, NP, false>), dim3(L.sc.n_pad), dim3(64 * PASS_WAVES), 0, s, L.args, L.sc);
+  const dim3 grid(L.sc.n_pad), block(64 * PASS_WAVES);
+  if (L.kappa == 2) hipLaunchKernelGGL((k_pass<MAT, NP, 2>), grid, block, 0, s, L.args, L.sc);
+  else if (L.kappa) hipLaunchKernelGGL((k_pass<MAT, NP, 1>), grid, block, 0, s, L.args, L.sc);
+  else hipLaunchKernelGGL((k_pass<MAT, NP, 0>), grid, block, 0, s, L.args, L.sc);
 }
 
 template <int MAT>

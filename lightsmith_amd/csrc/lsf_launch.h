@@ -55,7 +55,7 @@ struct PassArgs;
 struct PassLaunch {
   const PassArgs* args;  // device, one entry per member
   Sched sc;
-  int mat, np, kappa;
+  int mat, np, kappa;    // kappa: on no axis (0), on every axis with CPML (1), on some (2)
 };
 void launch_pass(const PassLaunch& L, hipStream_t s);
 // the D-form chunk table of an engine (n = 3 chunks of every row) from its E kernel arguments

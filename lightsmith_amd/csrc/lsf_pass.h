@@ -51,6 +51,7 @@ struct PassArgs {
   const float* psiHi[3][3];
   float* psiHo[3][3];
   int ns[2][3];
+  int has_k[2][3];            // the axis has the kappa term
   int zlo, zhi;               // planes [zlo, zhi) lie in no z slab
   const DChunk* dform;        // [N2][N1][nchunk][3]
   void* P;
@@ -100,7 +101,7 @@ __device__ __forceinline__ float hide(float x) {
 __device__ __forceinline__ cbytes in_bytes(const void* p) { return (cbytes)as_global((const char*)p); }
 __device__ __forceinline__ bytes out_bytes(void* p) { return (bytes)as_global((char*)p); }
 
-template <int MAT, int NP, bool KAP>
+template <int MAT, int NP, int KAP>
 __device__ __forceinline__ void tile(const PassArgs& a, int t, const float* tab, const float4* med, Nodes* nodes) {
   const Grid& g = a.g;
   const int lane = threadIdx.x & 63;
@@ -148,14 +149,15 @@ __device__ __forceinline__ void tile(const PassArgs& a, int t, const float* tab,
   const bytes G0 = out_bytes(a.H_out), G1 = G0 + comp, G2 = G1 + comp;
   const cbytes M0 = in_bytes(MAT == 1 ? (const void*)a.mid : (const void*)a.cbd), M1 = M0 + comp, M2 = M1 + comp;
 
-  // acc + the CPML term of one axis; psi advances. (The profile's c is hidden from the loop: its products with the
+  // acc + the CPML term of one axis; psi advances. KAP: no axis has the kappa term (0), every one with CPML (1) or some (2:
+  // asked for each, 1 % of a 131 x 117 x 150 box's step). (The profile's c is hidden from the loop: its products with the
   // coefficients would be kept in a register each.)
-  auto pml = [](float acc, const float4 pr, float coef, float der, float& psi) {
-    return acc + pml_apply(make_float4(pr.x, hide(pr.y), KAP ? hide(pr.z) : pr.z, pr.w), KAP, coef, der, psi);
+  auto pml = [](float acc, const float4 pr, int has_k, float coef, float der, float& psi) {
+    return acc + pml_apply(make_float4(pr.x, hide(pr.y), KAP ? hide(pr.z) : pr.z, pr.w), KAP == 1 || (KAP == 2 && has_k), coef, der, psi);
   };
   // the same along x or y, for the lanes in the slab
-  auto pml_in = [&](float acc, const float4 pr, float coef, float der, float& psi) {
-    const float v = pml(acc, pr, coef, der, psi);
+  auto pml_in = [&](float acc, const float4 pr, int has_k, float coef, float der, float& psi) {
+    const float v = pml(acc, pr, has_k, coef, der, psi);
     return pr.w >= 0.f ? v : acc;
   };
   // psi offsets: x slabs [k][j][p], y slabs [k][p][i], z slabs [p][j][i] (o: the cell's offset on plane k)
@@ -236,15 +238,15 @@ __device__ __forceinline__ void tile(const PassArgs& a, int t, const float* tab,
     {
       const float da = azu - az, db = y1 - ay;
       float acc = -cH * (da - db);
-      if (has_yh) acc = pml_in(acc, phy, -cH, da, qy);
-      if (iz >= 0) acc = pml(acc, pz, cH, db, qz0);
+      if (has_yh) acc = pml_in(acc, phy, a.has_k[1][1], -cH, da, qy);
+      if (iz >= 0) acc = pml(acc, pz, a.has_k[1][2], cH, db, qz0);
       hxq = hx + acc;
     }
     {
       const float azr = shfl_dn(az), da = x1 - ax, db = azr - az;
       float acc = -cH * (da - db);
-      if (has_xh) acc = pml_in(acc, phx, cH, db, qx);
-      if (iz >= 0) acc = pml(acc, pz, -cH, da, qz1);
+      if (has_xh) acc = pml_in(acc, phx, a.has_k[1][0], cH, db, qx);
+      if (iz >= 0) acc = pml(acc, pz, a.has_k[1][2], -cH, da, qz1);
       hyq = hy + acc;
     }
     o0 += plane;
@@ -331,14 +333,14 @@ __device__ __forceinline__ void tile(const PassArgs& a, int t, const float* tab,
       float acc = -cH * (da - db), acc0 = -cH * (da0 - db0);
       if (has_yh) {
         float n = qxy, n0 = qxy0;
-        acc = pml_in(acc, phy, -cH, da, n);
-        acc0 = pml_in(acc0, phy0, -cH, da0, n0);
+        acc = pml_in(acc, phy, a.has_k[1][1], -cH, da, n);
+        acc0 = pml_in(acc0, phy0, a.has_k[1][1], -cH, da0, n0);
         qxy = st ? n : qxy;
       }
       if (izh >= 0) {
         float n = qxz, n0 = qxz0;
-        acc = pml(acc, pzh, cH, db, n);
-        acc0 = pml(acc0, pzh, cH, db0, n0);
+        acc = pml(acc, pzh, a.has_k[1][2], cH, db, n);
+        acc0 = pml(acc0, pzh, a.has_k[1][2], cH, db0, n0);
         qxz = st ? n : qxz;
       }
       hx1 = st ? hx1 + acc : hx1;
@@ -350,12 +352,12 @@ __device__ __forceinline__ void tile(const PassArgs& a, int t, const float* tab,
       float acc = -cH * (da - db);
       if (has_xh) {
         float n = qyx;
-        acc = pml_in(acc, phx, cH, db, n);
+        acc = pml_in(acc, phx, a.has_k[1][0], cH, db, n);
         qyx = st ? n : qyx;
       }
       if (izh >= 0) {
         float n = qyz;
-        acc = pml(acc, pzh, -cH, da, n);
+        acc = pml(acc, pzh, a.has_k[1][2], -cH, da, n);
         qyz = st ? n : qyz;
       }
       hy1 = st ? hy1 + acc : hy1;
@@ -366,14 +368,14 @@ __device__ __forceinline__ void tile(const PassArgs& a, int t, const float* tab,
       float acc = -cH * (da - db), acc0 = -cH * (da0 - db0);
       if (has_xh) {
         float n = qzx, n0 = qzx0;
-        acc = pml_in(acc, phx, -cH, da, n);
-        acc0 = pml_in(acc0, phx, -cH, da0, n0);
+        acc = pml_in(acc, phx, a.has_k[1][0], -cH, da, n);
+        acc0 = pml_in(acc0, phx, a.has_k[1][0], -cH, da0, n0);
         qzx = st ? n : qzx;
       }
       if (has_yh) {
         float n = qzy, n0 = qzy0;
-        acc = pml_in(acc, phy, cH, db, n);
-        acc0 = pml_in(acc0, phy0, cH, db0, n0);
+        acc = pml_in(acc, phy, a.has_k[1][1], cH, db, n);
+        acc0 = pml_in(acc0, phy0, a.has_k[1][1], cH, db0, n0);
         qzy = st ? n : qzy;
       }
       hz1 = st ? hz1 + acc : hz1;
@@ -447,12 +449,12 @@ __device__ __forceinline__ void tile(const PassArgs& a, int t, const float* tab,
       float acc = c * (da - db);
       if (has_ye) {
         float n = sxy;
-        acc = pml_in(acc, pey, c, da, n);
+        acc = pml_in(acc, pey, a.has_k[0][1], c, da, n);
         sxy = st ? n : sxy;
       }
       if (ize >= 0) {
         float n = sxz;
-        acc = pml(acc, pze, -c, db, n);
+        acc = pml(acc, pze, a.has_k[0][2], -c, db, n);
         sxz = st ? n : sxz;
       }
       ex = finish(0, st, x1, acc);
@@ -463,12 +465,12 @@ __device__ __forceinline__ void tile(const PassArgs& a, int t, const float* tab,
       float acc = c * (da - db);
       if (has_xe) {
         float n = syx;
-        acc = pml_in(acc, pex, -c, db, n);
+        acc = pml_in(acc, pex, a.has_k[0][0], -c, db, n);
         syx = st ? n : syx;
       }
       if (ize >= 0) {
         float n = syz;
-        acc = pml(acc, pze, c, da, n);
+        acc = pml(acc, pze, a.has_k[0][2], c, da, n);
         syz = st ? n : syz;
       }
       ey = finish(1, st, y1, acc);
@@ -479,12 +481,12 @@ __device__ __forceinline__ void tile(const PassArgs& a, int t, const float* tab,
       float acc = c * (da - db);
       if (has_xe) {
         float n = szx;
-        acc = pml_in(acc, pex, c, da, n);
+        acc = pml_in(acc, pex, a.has_k[0][0], c, da, n);
         szx = st ? n : szx;
       }
       if (has_ye) {
         float n = szy;
-        acc = pml_in(acc, pey, -c, db, n);
+        acc = pml_in(acc, pey, a.has_k[0][1], -c, db, n);
         szy = st ? n : szy;
       }
       ew = finish(2, st, w1, acc);
@@ -556,7 +558,7 @@ __device__ __forceinline__ void tick_pair(const PassArgs& a, int lt) {
 
 }  // namespace pass
 
-template <int MAT, int NP, bool KAP>
+template <int MAT, int NP, int KAP>
 __global__ void __launch_bounds__(64 * PASS_WAVES) k_pass(const PassArgs* __restrict__ args, Sched sc) {
   __shared__ float tab[MAT == 1 ? 256 : 1];
   __shared__ float4 med_tab[NP > 0 ? MAX_MEDIA_VEC4 : 1];

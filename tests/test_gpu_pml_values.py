@@ -1,6 +1,6 @@
 """CPML values at their limits, every bulk kernel against the row kernels of another tile shape: an infinite or undefined psi
-reaches the cells that the update carries it to and no others. Single pass, lean, flat (real and complex) and adjoint
-kernels.
+reaches the cells that the update carries it to and no others; 1/kappa counts only where the axis was given with
+has_kappa. Single pass, lean, flat (real and complex) and adjoint kernels.
 """
 
 import numpy as np
@@ -62,3 +62,34 @@ def test_a_non_finite_psi_stays_with_its_cell(gpu, form, value):
             e.steps(3)
         _same(a, b, (form, block))
         assert torch.isfinite(a.E_flat.abs()).float().mean() > 0.9
+
+
+def _axes(e):
+    """(field, axis, profile, slab cells, psi) of the engine's CPML, as it gave them to the library."""
+    from lightsmith_amd.fdtd.engine import pml_axis_profile
+    spec = cases.product_ns().PMLSpec(cells=e.pml_cells, kappa_max=2.0, alpha_max=0.01)
+    state = iter(e._state)
+    for d in range(3):
+        if any(e.pml_cells[d]):
+            for f in range(2):
+                prof, ns, has_k = pml_axis_profile(spec, e.shape, e.dt, e.spacing, d, f)
+                yield f, d, prof, ns, has_k, next(state).view(2, -1)
+
+
+def _set(e, f, d, prof, ns, has_k, psi):
+    from lightsmith_amd import _lib
+    p = [_lib.ptr(psi[0 if c == min(q for q in range(3) if q != d) else 1]) if c != d else None for c in range(3)]
+    _lib.check(e.lib.lsf_set_pml(e._h, f, d, _lib.ptr(e.to_device(prof.astype(np.float32))), ns, *p, int(has_k)), "lsf_set_pml")
+
+
+@pytest.mark.parametrize("plain", [0, 1, 2])
+@pytest.mark.parametrize("form", FORMS)
+def test_kappa_is_skipped_on_an_axis_given_without(gpu, form, plain):
+    a, b = _engine(gpu, form), _engine(gpu, form, rows=True)
+    for e in (a, b):
+        for f, d, prof, ns, has_k, psi in _axes(e):
+            assert has_k
+            if d == plain:
+                _set(e, f, d, prof, ns, False, psi)
+        e.steps(5)
+    _same(a, b, (form, plain))
