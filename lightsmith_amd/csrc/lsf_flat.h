@@ -195,14 +195,15 @@ __device__ __forceinline__ void st_xpsi(bytes b, unsigned row, const XSlab<V>& s
     if (s.p[e] >= 0 && e >= sh) st1<T>(b, (row + (unsigned)s.p[e]) * (unsigned)sizeof(T), o[e]);
 }
 
-// acc += the CPML term of one axis, per cell (pml_apply's arithmetic); keep: psi keeps its old value there
+// acc += the CPML term of one axis, per cell in its slab (pml_apply's arithmetic); keep: psi keeps its old value there
 template <class T, int V>
 __device__ __forceinline__ void xterm(T (&acc)[V], const XSlab<V>& s, int has_k, float coef, const T (&der)[V],
                                       T (&psi)[V], bool keep0, bool keepl) {
 #pragma unroll
   for (int e = 0; e < V; ++e) {
     T pn = psi[e];
-    acc[e] = add(acc[e], pml_apply(s.pr[e], has_k, coef, der[e], pn));
+    const T v = add(acc[e], pml_apply(s.pr[e], has_k, coef, der[e], pn));
+    acc[e] = s.p[e] >= 0 ? v : acc[e];
     const bool keep = (e == 0 && keep0) || (e == V - 1 && keepl);
     psi[e] = keep ? psi[e] : pn;
   }
@@ -587,8 +588,8 @@ __device__ __forceinline__ void e_tile(const StepArgs& a, int t, const float* ta
 #pragma unroll
       for (int e = 0; e < V; ++e) {
         T pn = psi[e];
-        acc[e] = add(acc[e], pml_apply(xs.pr[e], a.pml[0].has_k,
-                                       cbe[e] * s, der[e], pn));
+        const T v = add(acc[e], pml_apply(xs.pr[e], a.pml[0].has_k, cbe[e] * s, der[e], pn));
+        acc[e] = xs.p[e] >= 0 ? v : acc[e];
         const bool keep = (e == 0 && kf[c]) || (e == V - 1 && kl);
         psi[e] = keep ? psi[e] : pn;
       }

@@ -1,6 +1,6 @@
 """CPML values at their limits, every bulk kernel against the row kernels of another tile shape: an infinite or undefined psi
-reaches the cells that the update carries it to and no others; 1/kappa counts only where the axis was given with
-has_kappa. Single pass, lean, flat (real and complex) and adjoint kernels.
+reaches the cells that the update carries it to and no others; a profile's b, c and 1/kappa count only inside its slab,
+and 1/kappa only where the axis was given with has_kappa. Single pass, lean, flat (real and complex) and adjoint kernels.
 """
 
 import numpy as np
@@ -80,6 +80,19 @@ def _set(e, f, d, prof, ns, has_k, psi):
     from lightsmith_amd import _lib
     p = [_lib.ptr(psi[0 if c == min(q for q in range(3) if q != d) else 1]) if c != d else None for c in range(3)]
     _lib.check(e.lib.lsf_set_pml(e._h, f, d, _lib.ptr(e.to_device(prof.astype(np.float32))), ns, *p, int(has_k)), "lsf_set_pml")
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_a_profile_counts_inside_its_slab_only(gpu, form):
+    a, b, ref = _engine(gpu, form), _engine(gpu, form, rows=True), _engine(gpu, form, rows=True)
+    for e in (a, b):
+        for f, d, prof, ns, has_k, psi in _axes(e):
+            prof[prof[:, 3] < 0, :3] = 1.0, 0.5, 0.25
+            _set(e, f, d, prof, ns, has_k, psi)
+    for e in (a, b, ref):
+        e.steps(5)
+    _same(b, ref, form)
+    _same(a, ref, form)
 
 
 @pytest.mark.parametrize("plain", [0, 1, 2])
