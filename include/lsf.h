@@ -199,7 +199,8 @@ int lsf_step(lsf_engine* eng, int n_steps, void* stream);
  * that lsf_step keeps in a library allocation are staged instead, on `stream`, in one file-scope device array of
  * 8 KiB per GPU, shared by every call on that GPU: calls that overlap on one GPU (other streams or host threads)
  * race. Refused with an error: engines with sub-engines (their arguments exceed the array) and engines set to
- * single-pass stepping by lsf_set_fused. */
+ * single-pass stepping by lsf_set_fused: real fields without periodic axes, one row per lane and 64 x cells per row,
+ * nothing between the H and the E update, 12 * cells < 2^32. */
 int lsf_step_noalloc(lsf_engine* eng, int n_steps, void* stream);
 /* As lsf_step, bracketing each H and E kernel with HIP events on `stream`; adds the summed kernel times (ms)
  * to ms[0] (H kernels) and ms[1] (E kernels; the single-pass kernel when the engine steps with it, ms[0] then
@@ -283,13 +284,13 @@ int lsf_batch_graph_reset(lsf_batch* batch);
 /* Single-pass stepping (no reference counterpart: a launch choice). dev_E2, dev_H2: a second set of field buffers;
  * dev_psiH2[axis]: a second set of the H-side psi arrays of each axis with CPML (null where none), laid out like the
  * first, whose two component arrays must be contiguous (the second component's array right after the first's). Their
- * contents do not matter. Where the engine allows it -- real fields, no periodic axes, one row per lane and four
- * wavefronts per block, no operations between the H and the E update except a design tape -- steps are then run two
+ * contents do not matter. Where the engine allows it -- real fields, cubic cells, no periodic axes, one row per lane and
+ * four wavefronts per block, no operations between the H and the E update except a design tape -- steps are then run two
  * at a time, each one kernel that reads one set and writes the other; an odd last step runs the H and the E kernel in
  * place. So dev_E, dev_H and the first psi arrays hold the state whenever the host has control, and lsf_parity is
  * always 0. Results are bit-identical to the two-kernel step. lsf_can_pair: whether the engine as configured so far
- * could step this way (0: no; 1: yes, but the two kernels are the faster step; 2: yes, and faster). lsf_set_fused is lsf_set_pair for a caller that requires it: lsf_step_noalloc
- * then refuses the engine. */
+ * could step this way (0: no; 1: yes, but the two kernels are the faster step; 2: yes, and faster). lsf_set_fused is
+ * lsf_set_pair for a caller that asks for it: lsf_step_noalloc then refuses the engine. */
 int lsf_set_pair(lsf_engine* eng, void* dev_E2, void* dev_H2, void* const* dev_psiH2);
 int lsf_can_pair(lsf_engine* eng);
 int lsf_set_fused(lsf_engine* eng, void* dev_E2, void* dev_H2, void* const* dev_psiH2);

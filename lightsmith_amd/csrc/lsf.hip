@@ -335,11 +335,11 @@ bool has_h_phase_ops(const lsf_engine* e) {
   return false;
 }
 
-// elements from the first to the second H-side psi array of an axis when they are contiguous, else -1
-long long psi_gap(const lsf_engine* e, int ax) {
+// elements from the first to the second psi array of a field (H: of the first set) and axis when they are contiguous, else -1
+long long psi_gap(const lsf_engine* e, int field, int ax) {
   const int c1 = ax == 0 ? 1 : 0, c2 = ax == 2 ? 1 : 2;
-  void* const* ps = e->psiH[0][ax];
-  long long size = e->pml[1][ax].ns;
+  void* const* ps = field ? e->psiH[0][ax] : e->pml[0][ax].psi;
+  long long size = e->pml[field][ax].ns;
   for (int a = 0; a < 3; ++a)
     if (a != ax) size *= e->g.n[a];
   if (!ps[c1] || !ps[c2]) return -1;
@@ -362,6 +362,20 @@ bool pass_eligible(const lsf_engine* e) {
     }
   }
   return e->g.N < (1ll << 30);
+}
+
+// Whether an engine was asked to step in single passes (lsf_set_fused) and is of the form that the request is for: real
+// fields without periodic axes, one-row tiles of 64 cells, nothing between the H and the E update, fields within 32-bit
+// offsets, contiguous psi. lsf_step_noalloc refuses these, also where lsf_step takes two kernels.
+bool fused_form(const lsf_engine* e) {
+  if (!e->asked_fused || e->cplx || any_periodic(e) || e->adjoint || e->ry != 1 || e->xw != 64 || 12 * e->g.N >= (1ll << 32))
+    return false;
+  for (const Op& o : e->ops)
+    if (o.phase <= LSF_PH_ADVANCE_H || o.phase == LSF_PH_BEFORE_H) return false;
+  for (int f = 0; f < 2; ++f)
+    for (int ax = 0; ax < 3; ++ax)
+      if (e->pml[f][ax].prof && psi_gap(e, f, ax) < 0) return false;
+  return true;
 }
 
 long long second_bytes(const lsf_engine* e) {  // the second set of a pass
@@ -1725,7 +1739,7 @@ int lsf_step_noalloc(lsf_engine* e, int n, void* stream) {
     if (o.kind == OP_SUB_H)
       return fail(LSF_EINVAL, "lsf_step_noalloc: an engine with sub-engines needs more kernel-argument scratch "
                               "than the 8 KiB it holds; use lsf_step");
-  if (e->asked_fused && pass_eligible(e))
+  if (fused_form(e))
     return fail(LSF_EINVAL, "lsf_step_noalloc: single-pass stepping is not supported; use lsf_step");
   const size_t need = 2 * sizeof(StepArgs);
   if (need > kNoAllocScratchBytes) return fail(LSF_EINVAL, "lsf_step_noalloc: kernel arguments exceed the scratch");
@@ -1911,7 +1925,7 @@ int lsf_set_pair(lsf_engine* e, void* E2, void* H2, void* const* psiH2) {
     for (int c = 0; c < 3; ++c) e->psiH[1][ax][c] = nullptr;
     if (!e->pml[1][ax].prof) continue;
     if (!psiH2 || !psiH2[ax]) return fail(LSF_EINVAL, "missing second H-side psi set");
-    const long long gap = psi_gap(e, ax);
+    const long long gap = psi_gap(e, 1, ax);
     if (gap < 0) return fail(LSF_EINVAL, "the H-side psi arrays of an axis must be contiguous");
     const int c1 = ax == 0 ? 1 : 0, c2 = ax == 2 ? 1 : 2;
     e->psiH[1][ax][c1] = psiH2[ax];

@@ -414,7 +414,9 @@ class Engine:
             return
         self._pair_open = False
         can = self.lib.lsf_can_pair(self._h)  # 1: it could, 2: and it is the faster step
-        if not (can if self._fused else can == 2 and Engine.single_pass):
+        # a request holds for these forms whether or not the pass can step them (lsf_step_noalloc refuses them)
+        form = not self.complex and not any(self.periodic) and self.tiling[0] == 1 and self.tiling[2] == 64
+        if not (can or form if self._fused else can == 2 and Engine.single_pass):
             return
         try:
             sets = [torch.empty_like(self.E_flat), torch.empty_like(self.H_flat)] + \

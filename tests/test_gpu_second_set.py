@@ -1,0 +1,48 @@
+"""The second buffer set of single-pass stepping: who is given one and what is refused with it."""
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from tests import cases
+from tests.test_zz_no_alloc import _bind
+
+pytestmark = pytest.mark.gpu
+
+
+def _box(gpu, shape=(24, 20, 18), dx=2.0, tiling=None, **kw):
+    ns = cases.product_ns()
+    d = np.broadcast_to(dx, 3)
+    old = ns.Engine.tiling
+    ns.Engine.tiling = tiling or old
+    try:
+        e = cases.make(ns, gpu, shape=shape, dx=dx, dt=0.9 / np.sqrt(sum(1 / v ** 2 for v in d)),
+                       inv_eps=np.full((3,) + shape, 1 / 2.25), pml=ns.PMLSpec(cells=((3, 3),) * 3), **kw)
+    finally:
+        ns.Engine.tiling = old
+    cases.random_fields(e, 2)
+    return e
+
+
+@pytest.mark.parametrize("dx,tiling,refused", [(2.0, None, True), ((2.0, 1.5, 3.0), None, True), (2.0, (1, 8, 64, 8), True),
+                                               (2.0, (2, 4, 64, 8), False), (2.0, (1, 4, 32, 8), False)])
+def test_no_alloc_steps_refuse_what_was_asked_to_step_in_single_passes(gpu, dx, tiling, refused):
+    """fused=True on one-row tiles of 64 cells; other tiles, and engines that were not asked, are stepped."""
+    from lightsmith_amd import _lib
+    lib = _lib.load()
+    noalloc = _bind(lib)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for fused in (True, None):
+        a, b = (_box(gpu, dx=dx, tiling=tiling, fused=f) for f in (fused, False))
+        rc = noalloc(a._h, 3, stream)
+        if fused and refused:
+            assert rc == _lib.LSF_EINVAL and b"single-pass" in lib.lsf_last_error()
+            a.steps(3)
+        else:
+            assert rc == 0
+        b.steps(3)
+        torch.cuda.synchronize()
+        for x, y in zip(a.state_tensors(), b.state_tensors()):
+            assert torch.equal(x, y)
