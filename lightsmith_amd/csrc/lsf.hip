@@ -348,7 +348,7 @@ long long psi_gap(const lsf_engine* e, int field, int ax) {
 
 // Whether the single pass can step an engine: real fields on cubic cells, no periodic axes, the boxes of a grid without
 // mirror planes, no work between the H and the E update, a one-row, four-wavefront tile shape (the default and what the
-// drivers choose; another shape asks for the row kernels) and components below 4 GB (32-bit offsets).
+// drivers choose; another shape asks for the row kernels) and arrays below 4 GB (32-bit offsets).
 bool pass_eligible(const lsf_engine* e) {
   if (!e->pair_set || !e->tick || e->cplx || any_periodic(e) || e->adjoint || e->ry != 1 || e->waves != lsf::PASS_WAVES ||
       has_h_phase_ops(e))
@@ -361,7 +361,10 @@ bool pass_eligible(const lsf_engine* e) {
       if (e->g.rH[c][ax][0] != 0 || e->g.rH[c][ax][1] != (ax == c ? n : n - 1)) return false;
     }
   }
-  return e->g.N < (1ll << 30);
+  if (e->g.N >= (1ll << 30)) return false;
+  // the D-form chunk table, 3 chunks to 32 cells of a row: past 4 GB before a component is on rows of a few cells
+  const long long chunks = 3ll * ((e->g.n[0] + 31) / 32) * e->g.n[1] * e->g.n[2];
+  return pole_regs(e) == 0 || chunks * (long long)sizeof(lsf::DChunk) < (1ll << 32);
 }
 
 // Whether an engine was asked to step in single passes (lsf_set_fused) and is of the form that the request is for: real

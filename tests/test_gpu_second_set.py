@@ -46,3 +46,24 @@ def test_no_alloc_steps_refuse_what_was_asked_to_step_in_single_passes(gpu, dx, 
         torch.cuda.synchronize()
         for x, y in zip(a.state_tensors(), b.state_tensors()):
             assert torch.equal(x, y)
+
+
+def test_chunk_offsets_past_four_gigabytes_do_not_step_in_single_passes(gpu):
+    """D-form nodes on a grid a few cells wide: 24 bytes a chunk of 32 cells and row pass 2^32 before a component does. (Only asked:
+    the handle's arrays are never used.)"""
+    from lightsmith_amd import _lib
+    lib = _lib.load()
+    word = torch.zeros(64, dtype=torch.float32, device=gpu)
+    media = torch.tensor([1.0, 1.0, 0.5, 0.1, 0.2], device=gpu)
+    for shape, ok in (((3, 15000, 13000), 0), ((3, 9000, 13000), 2), ((40, 4000, 4000), 2)):
+        g = _lib.LsfGrid()
+        g.shape[:], g.spacing[:], g.dt, g.tick = shape, (2.0,) * 3, 1.0, 1
+        g.dev_E = g.dev_H = g.dev_counter = word.data_ptr()
+        h = ctypes.c_void_p()
+        _lib.check(lib.lsf_create(ctypes.byref(g), ctypes.byref(h)), "lsf_create")
+        _lib.check(lib.lsf_set_material_dense(h, _lib.ptr(word)), "lsf_set_material_dense")
+        _lib.check(lib.lsf_set_tiling(h, 1, 4, 64, 8), "lsf_set_tiling")
+        assert lib.lsf_can_pair(h) == 2
+        _lib.check(lib.lsf_set_ade(h, _lib.ptr(word), _lib.ptr(word), 10, 1, _lib.ptr(media), 1), "lsf_set_ade")
+        assert lib.lsf_can_pair(h) == ok, shape
+        lib.lsf_destroy(h)
