@@ -474,12 +474,26 @@ int plan_z(lsf_engine* e) {
   return rc;
 }
 
-// Arguments of the single pass, and the D-form chunk table.
+// Memory that a faster step wants and another one does without; null where there is no room for it.
+template <class P>
+int optional_malloc(P** p, size_t bytes, const char* what) {
+  const hipError_t got = hipMalloc(p, bytes);
+  if (got != hipErrorOutOfMemory) return hip_check(got, what);
+  (void)hipGetLastError();
+  *p = nullptr;
+  return LSF_OK;
+}
+
+// Arguments of the single pass, and the D-form chunk table; without room for that the two kernels step.
 int sync_pass(lsf_engine* e, const StepArgs& ea) {
   int rc = LSF_OK;
   if (pole_regs(e) > 0) {
     const long long n = 3ll * ea.nchunk * e->g.n[1] * e->g.n[2];
-    if (!e->dform) rc = hip_check(hipMalloc(&e->dform, sizeof(lsf::DChunk) * n), "hipMalloc D-form chunk table");
+    if (!e->dform) rc = optional_malloc(&e->dform, sizeof(lsf::DChunk) * n, "hipMalloc D-form chunk table");
+    if (!rc && !e->dform) {
+      e->use_pass = false;
+      return LSF_OK;
+    }
     if (!rc) rc = hip_check(hipDeviceSynchronize(), "synchronize before the D-form chunk table");
     if (rc) return rc;
     lsf::launch_dform_chunks(ea, e->dform, n, nullptr);
@@ -649,7 +663,8 @@ int plan_corr(lsf_engine* e) {
       }
       if (!ok) break;
       int* d = nullptr;
-      if ((rc = hip_check(hipMalloc(&d, sizeof(int) * row.size()), "hipMalloc correction rows"))) return rc;
+      if ((rc = optional_malloc(&d, sizeof(int) * row.size(), "hipMalloc correction rows"))) return rc;
+      if (!d) break;
       e->corr_rows.push_back(d);
       if ((rc = hip_check(hipMemcpy(d, row.data(), sizeof(int) * row.size(), hipMemcpyHostToDevice), "correction rows"))) return rc;
       lsf::Corr& q = cs.c[cs.n++];
@@ -851,8 +866,8 @@ int sync_args(lsf_engine* e) {
   }
   e->joined = mem.size() > 1;
   e->use_pass = pass_eligible(e);
-  if ((rc = plan_stages(e))) return rc;
   if (e->use_pass && (rc = sync_pass(e, h[0]))) return rc;
+  if ((rc = plan_stages(e))) return rc;
   e->dirty = false;
   return LSF_OK;
 }

@@ -418,15 +418,16 @@ class Engine:
         form = not self.complex and not any(self.periodic) and self.tiling[0] == 1 and self.tiling[2] == 64
         if not (can or form if self._fused else can == 2 and Engine.single_pass):
             return
+        # one allocation, of parts of whole 512 bytes: where not all of it fits, none of it stays reserved
+        n = [-(-v // 128) * 128 for v in (self.E_flat.numel(), self.H_flat.numel(), *self._psiH_size)]
         try:
-            sets = [torch.empty_like(self.E_flat), torch.empty_like(self.H_flat)] + \
-                [torch.empty(n, dtype=self.fdt, device=self._dev) if n else None for n in self._psiH_size]
+            sets = torch.empty(sum(n), dtype=self.fdt, device=self._dev).split(n)
         except torch.cuda.OutOfMemoryError:  # the two-kernel step needs no second set
             if self._fused:
                 raise
             return
-        self._keep += [t for t in sets if t is not None]
-        arr = (ctypes.c_void_p * 3)(*[None if t is None else t.data_ptr() for t in sets[2:]])
+        self._keep += sets
+        arr = (ctypes.c_void_p * 3)(*[t.data_ptr() if t.numel() else None for t in sets[2:]])
         give = self.lib.lsf_set_fused if self._fused else self.lib.lsf_set_pair
         check(give(self._h, ptr(sets[0]), ptr(sets[1]), arr), "lsf_set_pair")
         self._two_sets = True

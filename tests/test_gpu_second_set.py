@@ -1,4 +1,4 @@
-"""The second buffer set of single-pass stepping: who is given one and what is refused with it."""
+"""The second buffer set of single-pass stepping: who is given one, what is refused with it, and a GPU without room for it."""
 
 import ctypes
 
@@ -67,3 +67,24 @@ def test_chunk_offsets_past_four_gigabytes_do_not_step_in_single_passes(gpu):
         _lib.check(lib.lsf_set_ade(h, _lib.ptr(word), _lib.ptr(word), 10, 1, _lib.ptr(media), 1), "lsf_set_ade")
         assert lib.lsf_can_pair(h) == ok, shape
         lib.lsf_destroy(h)
+
+
+def test_without_room_the_second_set_leaves_nothing_behind(gpu):
+    """Where not all of it fits, the engine steps with two kernels and holds no part of it, and one that asked for it raises."""
+    a, b = _box(gpu, shape=(260, 256, 256)), _box(gpu, shape=(260, 256, 256), fused=False)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    held = torch.cuda.memory_reserved(gpu)
+    total = torch.cuda.get_device_properties(gpu).total_memory
+    torch.cuda.set_per_process_memory_fraction((held + 1.5 * 4 * a.E_flat.numel()) / total, gpu)  # room for one field of two
+    try:
+        a.steps(2)
+        b.steps(2)
+        assert not a._two_sets and torch.cuda.memory_reserved(gpu) == held
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            _box(gpu, shape=(260, 256, 256), fused=True)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, gpu)
+    torch.cuda.synchronize()
+    for x, y in zip(a.state_tensors(), b.state_tensors()):
+        assert torch.equal(x, y)
