@@ -15,7 +15,7 @@ import torch
 
 from .. import _lib
 from .._lib import check
-from .engine import Engine
+from .engine import CallerStream, Engine
 
 # tile shapes with compiled kernels: (rows per lane, wavefronts per block, x cells per wavefront row)
 SHAPES = ((1, 4, 64), (2, 4, 64), (1, 8, 64), (2, 8, 64), (1, 4, 32), (2, 4, 32), (1, 8, 32), (2, 8, 32))
@@ -140,7 +140,8 @@ class Batch:
             return self.chunk, False
         stream = torch.cuda.Stream(device=self._dev)
         stream.wait_stream(torch.cuda.current_stream(self._dev))
-        state = {"captured": False, "last": None}
+        state = {"captured": False}
+        caller = CallerStream(self._dev)
         self._graph_stream = stream
 
         def run():
@@ -152,11 +153,8 @@ class Batch:
                 state["captured"] = True
                 self._graphed = True
                 return
-            cur = torch.cuda.current_stream(self._dev)  # on the caller's stream, as Engine.make_runner
-            if state["last"] is not None and state["last"] != cur:
-                cur.wait_stream(state["last"])
-            state["last"] = cur
-            check(self.lib.lsf_batch_graph_replay(self._h, 1, ctypes.c_void_p(cur.cuda_stream)), "lsf_batch_graph_replay")
+            check(self.lib.lsf_batch_graph_replay(self._h, 1, caller.begin()), "lsf_batch_graph_replay")
+            caller.end()
             self._advance(self.stride)
 
         return run, True

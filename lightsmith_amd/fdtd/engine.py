@@ -283,6 +283,29 @@ def _device_of(device) -> torch.device:
     return dev
 
 
+class CallerStream:
+    """Work launched on the caller's stream, call after call: a stream other than the last one waits for it, as the replays of
+    one graph follow one another. (Replays on a side stream cost two event waits a chunk.) Torch's own streams live as long
+    as the process; one that it only wraps may be gone by the next call, so the end of the work there is kept in an event
+    (5 us a chunk: 73.7 -> 78.5 us on a 40 x 36 x 32 box)."""
+
+    def __init__(self, dev):
+        self._dev, self._last, self._event = dev, None, None
+
+    def begin(self):
+        cur = torch.cuda.current_stream(self._dev)
+        if self._event is not None:
+            cur.wait_event(self._event)
+        elif self._last is not None and self._last != cur:
+            cur.wait_stream(self._last)
+        self._last = cur
+        return ctypes.c_void_p(cur.cuda_stream)
+
+    def end(self):
+        wrapped = self._last.cuda_stream != 0 and self._last.stream_id == self._last.cuda_stream
+        self._event = self._last.record_event() if wrapped else None
+
+
 class Engine:
     """FDTD engine whose stepping runs in the HIP library (engine.py:230-315 constructor contract)."""
 
@@ -905,7 +928,8 @@ class Engine:
             return self.chunk, False
         stream = torch.cuda.Stream(device=self._dev)
         stream.wait_stream(torch.cuda.current_stream(self._dev))
-        state = {"captured": False, "last": None}
+        state = {"captured": False}
+        caller = CallerStream(self._dev)
         self._graph_stream = stream
 
         def run():
@@ -917,13 +941,8 @@ class Engine:
                 state["captured"] = True
                 self._graphed = True
                 return
-            # replayed on the caller's stream: a side stream costs two event waits a chunk. A stream other than the last
-            # one waits for it, as the replays of one graph follow one another.
-            cur = torch.cuda.current_stream(self._dev)
-            if state["last"] is not None and state["last"] != cur:
-                cur.wait_stream(state["last"])
-            state["last"] = cur
-            check(self.lib.lsf_graph_replay(self._h, 1, ctypes.c_void_p(cur.cuda_stream)), "lsf_graph_replay")
+            check(self.lib.lsf_graph_replay(self._h, 1, caller.begin()), "lsf_graph_replay")
+            caller.end()
             self.n_host += self.stride
 
         return run, True
