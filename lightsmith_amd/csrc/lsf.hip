@@ -581,11 +581,8 @@ int make_sched(const std::vector<int>& counts, lsf::Sched* sc, std::vector<void*
   return rc;
 }
 
-// Give the leading gathers and modal sources that follow a field's update to the bulk kernel (Corr). An operation stays a
-// launch, and those behind it with it, where its rows repeat a node or name one that does not step, read what the bulk
-// kernel writes, or lie so thin in their box that the table would outgrow them (more than 16 entries a row), and past
-// MAX_CORR; so do all behind an off-diagonal gather.
-std::vector<Op*> in_order(lsf_engine* e, int field) {  // what runs after a field's update
+// What runs after a field's update, in order.
+std::vector<Op*> in_order(lsf_engine* e, int field) {
   std::vector<Op*> v;
   for (int ph = field ? LSF_PH_CORRECT_H : LSF_PH_OFFDIAG; ph <= (field ? LSF_PH_ADVANCE_H : LSF_PH_ADVANCE_E); ++ph)
     for (Op& o : e->ops)
@@ -593,6 +590,10 @@ std::vector<Op*> in_order(lsf_engine* e, int field) {  // what runs after a fiel
   return v;
 }
 
+// Give the leading gathers and modal sources that follow a field's update to the bulk kernel (Corr). An operation stays a
+// launch, and those behind it with it, where its rows repeat a node or name one that does not step, read what the bulk
+// kernel writes, or lie so thin in their box that the table would outgrow them (more than 16 entries a row), past
+// MAX_CORR or where there is no room for its table; so do all behind an off-diagonal gather.
 int plan_corr(lsf_engine* e) {
   if (e->corr_planned) return LSF_OK;
   int rc = LSF_OK;
