@@ -1,6 +1,7 @@
 """The second buffer set of single-pass stepping: who is given one, what is refused with it, and a GPU without room for it."""
 
 import ctypes
+import gc
 
 import numpy as np
 import pytest
@@ -73,9 +74,17 @@ def test_without_room_the_second_set_leaves_nothing_behind(gpu):
     """Where not all of it fits, the engine steps with two kernels and holds no part of it, and one that asked for it raises."""
     a, b = _box(gpu, shape=(260, 256, 256)), _box(gpu, shape=(260, 256, 256), fused=False)
     torch.cuda.synchronize()
+    gc.collect()
     torch.cuda.empty_cache()
     held = torch.cuda.memory_reserved(gpu)
     total = torch.cuda.get_device_properties(gpu).total_memory
+    torch.cuda.set_per_process_memory_fraction(held / total, gpu)
+    kept = []  # reserved memory that would do
+    try:
+        while True:
+            kept.append(torch.empty(2 * a.E_flat.numel(), device=gpu))
+    except torch.cuda.OutOfMemoryError:
+        held = torch.cuda.memory_reserved(gpu)
     torch.cuda.set_per_process_memory_fraction((held + 1.5 * 4 * a.E_flat.numel()) / total, gpu)  # room for one field of two
     try:
         a.steps(2)
