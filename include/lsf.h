@@ -67,7 +67,8 @@ int lsf_set_material_indexed(lsf_engine* eng, const uint32_t* dev_ids, const flo
  * applied in _update_H/_update_E (engine.py:344-418, 636-643, 656-663).
  * dev_profile[shape[axis]] float4 = {b, c, 1/kappa, slab index (or -1)} at each node position along the axis;
  * dev_psi[c] (c != axis) = the psi array of component c, slab extent n_slab along the axis, full extent
- * along the other two (field type). has_kappa = 0 skips the kappa term as the reference does. */
+ * along the other two (field type). has_kappa = 0 skips the kappa term as the reference does. The slab indices of the z
+ * profiles are read when the engine first steps after a configuration call, the rest at every step. */
 int lsf_set_pml(lsf_engine* eng, int field, int axis, const void* dev_profile, int n_slab, void* dev_psi0,
                 void* dev_psi1, void* dev_psi2, int has_kappa);
 
@@ -80,7 +81,9 @@ int lsf_set_pml(lsf_engine* eng, int field, int axis, const void* dev_profile, i
  * (dE - sum (P^{n+1} - P^n)) / eps_inf. dev_media[n_media][2 + 3*max_poles] float =
  * {1/eps_inf, n_poles, (c1, c2, c3) per pole} (pole_coefficients, engine.py:108-111), zeros for the poles past a
  * medium's n_poles (the E kernel advances max_poles poles for every node; zero coefficients keep those poles at
- * zero); n_media * (2 + 3*max_poles) <= 224 (16 media of 4 poles, 44 of 1). */
+ * zero); n_media * (2 + 3*max_poles) <= 224 (16 media of 4 poles, 44 of 1). Which nodes are in D-form (the material's
+ * negative entries) and dev_chunk_base are read when the engine first steps after a configuration call; other values of
+ * the material may be changed in place between steps. */
 int lsf_set_ade(lsf_engine* eng, const int32_t* dev_chunk_base, void* dev_P, int64_t n_nodes, int max_poles,
                 const float* dev_media, int n_media);
 
@@ -183,7 +186,9 @@ int lsf_set_energy(lsf_engine* eng, float* dev_energy);
 
 /* Launch tuning: rows per lane (1 or 2), wavefronts per block (4 or 8), x cells per wavefront row (64: one
  * row per wavefront; 32: two rows), z planes per block (>= 1; the E kernel of an engine with pole state marches
- * twice as many). No reference counterpart (a launch choice). */
+ * twice as many). At one row and four wavefronts the kernels that lay a plane's rows end to end step the engine where they
+ * can (single passes, engines with a periodic axis, adjoint ones, most without poles); these choose their own planes
+ * per block, and x_cells and z_chunk are then only what the rest takes. No reference counterpart (a launch choice). */
 int lsf_set_tiling(lsf_engine* eng, int rows_per_lane, int waves, int x_cells, int z_chunk);
 
 /* Order of the E launch's tiles: reverse_e = 1 (the default) walks each XCD's contiguous tile range from its end,
@@ -258,15 +263,15 @@ int lsf_add_adjoint_source(lsf_engine* eng, int h_side, int nf, int64_t n_pts, c
  * No reference counterpart: the reference runs the angles/wavelengths/polarisations of an oblique sweep
  * one Engine after another (periodic.py:503-519). A batch steps its members with shared launches: per
  * half-step one bulk-kernel launch per kernel configuration over all members' tiles (one block per tile,
- * or a persistent grid that strides over them), each phase's per-step operations fused by position over
- * the members (gathers and modal sources one launch each, sub-engines as a nested batch), and one DFT
- * launch per source type for all monitors. Members are fully configured top-level engines with their own
+ * or a persistent grid that strides over them), the per-step operations of a stretch between bulk updates fused by
+ * stage over the members (gathers, modal sources and the small per-row jobs one launch each, sub-engines as a nested
+ * batch), and one DFT launch per source type for all monitors. Members are fully configured top-level engines with their own
  * step counters; while the batch exists they refuse configuration calls. Destroy the batch before its
  * members. Each member's state evolves exactly as under lsf_step / lsf_chunk of that member alone. */
 typedef struct lsf_batch lsf_batch;
 int lsf_batch_create(lsf_engine* const* members, int n_members, lsf_batch** out);
 void lsf_batch_destroy(lsf_batch* batch);
-/* Tile shape as lsf_set_tiling, for all members' bulk kernels; grid_blocks = 0 launches one block per tile,
+/* Tile shape as lsf_set_tiling, for all members' bulk kernels (a new batch starts at 2, 4, 64, 16); grid_blocks = 0 launches one block per tile,
  * grid_blocks > 0 a persistent grid of that many blocks (rounded up to a multiple of 8). */
 int lsf_batch_set_schedule(lsf_batch* batch, int rows_per_lane, int waves, int x_cells, int z_chunk,
                            int grid_blocks);

@@ -10,6 +10,9 @@
 // 64-bit base of the plane plus a fixed 32-bit lane offset: no address arithmetic in the loop. A row's last lane
 // starts at nx - V when V does not divide nx: it overlaps its neighbour, computes the shared cells again and stores
 // only its own, so every load is in bounds and V wide.
+// What is left: waits for memory (57-72 % of the wavefronts' time, 3.4 of them per SIMD for the registers of complex cells),
+// the vector units busy for 23-36 % of the cycles; 4.6-4.9 TB/s on one 76 x 61 x 256 complex cell, 5.4 (E) and 6.2 (H) on the
+// complex members of 12 as a batch.
 // Measured (complex64), row kernels -> these: one 76 x 61 x 256 cell 114 -> 63 us per step, its 3 x 3 column's launches
 // included; 12 cells of 50-98 x 50-98 x 256 as one batch 847 -> 520 us per step. One cell per lane: 60 against 55 us on
 // the first, 521 against 515 us on the second.

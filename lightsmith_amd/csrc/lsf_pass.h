@@ -14,8 +14,10 @@
 //
 // What bounds it. Two launches move E and H three times between them (72 B per cell and step and the coefficients), the
 // pass moves each once in and once out (48 B); its re-reads of neighbouring rows and planes are served by the caches.
-// Small and middling grids are then bound by instructions: 76 % of the vector issue cycles of a 192 x 160 x 128 box with
-// one-pole nodes hold one (265 a cell, D-form rounds and slabs included). So:
+// Past the memory-side cache that is HBM (320^3, 3 poles: 2.73 GB a step at 4.4 TB/s, the vector units busy for 37 % of the
+// cycles, 270 instructions a cell); within it the step's bytes move at 5.1-5.4 TB/s and instructions weigh as much: the
+// vector units are busy for 70 % of a 131 x 117 x 150 box's cycles (dense coefficients, kappa, 45 % of the cells in slabs:
+// 355 a cell) and for 54 % of a 192 x 160 x 128 one's with one-pole nodes (276 a cell). So:
 // - every address is a wave-uniform base and a 32-bit lane offset; the three row offsets advance by a plane per
 //   iteration (a component is below 4 GB), nothing else is recomputed;
 // - lanes outside a CPML slab read a psi that they do not use, whole wavefronts outside one skip its terms;

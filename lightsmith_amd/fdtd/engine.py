@@ -310,12 +310,13 @@ class Engine:
     """FDTD engine whose stepping runs in the HIP library (engine.py:230-315 constructor contract)."""
 
     # launch tiling (rows per lane, wavefronts per block, x cells per wavefront row, z planes per block; the E
-    # kernel of an engine with pole state marches twice the z planes); see lsf_set_tiling
+    # kernel of an engine with pole state marches twice the z planes); see lsf_set_tiling, also for the kernels that
+    # choose their own z planes
     tiling = (1, 4, 64, 8)
     # launch the tensor nodes' D update with the E-side table correction when their nodes are disjoint
     fuse_sparse = True
     # default of the `fused` argument: step eligible engines (real fields, no periodic axes, a one-row four-wavefront
-    # tile shape, no H-phase operations) in pairs of single passes over a second buffer set where that is faster
+    # tile shape, cubic cells, no H-phase operations) in pairs of single passes over a second buffer set where that is faster
     single_pass = True
 
     def __init__(self, device=None, *, shape, dx, dt: float, single: bool = True, inv_eps: np.ndarray,
